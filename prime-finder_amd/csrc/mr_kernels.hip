@@ -18,6 +18,7 @@
 // multiplies by the base, which is below 2^24, by double-and-add of modular
 // additions instead of a transform product.
 #include "mr_core.h"
+#include "mr_dec.h"
 #include "../../include/mr_gpu.h"
 
 #include <stdio.h>
@@ -62,6 +63,14 @@ struct Dev {                    // per-batch device state (kernel argument)
     uint8_t *alive;             // [n]
     uint8_t *pre;               // [n] 0 = test, 1 = prime (2, 3), 2 = composite (even, < 2)
     uint32_t *err;              // [1] error latch
+    // base-10^13 exponentiation of search-form numbers (mr_dec.h); nullptr:
+    // not for this context
+    dec::Form *form;            // [n]
+    int32_t *path;              // [n] class of the round in progress, 0: Montgomery step
+    double *dig;                // [n][dstride] the residue's digits (path != 0)
+    int dstride;
+    double *decNt, *park;       // [n][tstride], [n][pstride]: see dec::Args
+    int tstride, pstride;
 };
 
 __device__ __forceinline__ int slot_id(const Dev &D)
@@ -544,19 +553,20 @@ __device__ __forceinline__ void montmul(Smem<LOGM> &sm, const Twiddles &T, const
     reduce_once<C>(r, Nl, L, L, sm.sc, D.Nh + (size_t)c * M);
 }
 
-// x <- x * s (plain integer product), 1 <= s < 2^24.
+// x <- x * s + add (plain integers), 1 <= s < 2^24, add < 2^46.
 template <int C>
-__device__ __forceinline__ void mul_small_vec(uint32_t (&x)[C], uint32_t s, Scratch &sc)
+__device__ __forceinline__ void mul_small_vec(uint32_t (&x)[C], uint32_t s, Scratch &sc,
+                                              uint64_t add = 0)
 {
     const int t = tid_();
-    uint64_t acc = 0;
+    uint64_t acc = t ? 0ull : add;
 #pragma unroll
     for (int i = 0; i < C; i++) {
         acc += (uint64_t)x[i] * s;
         x[i] = (uint32_t)acc & LIMB_MASK;
         acc >>= LIMB_BITS;
     }
-    sc.carry[t] = acc;                  // < 2^24 + 2
+    sc.carry[t] = acc;                  // < 2^24 + 2 (+ 2^22 from add)
     lds_barrier();
     uint64_t cin = t ? sc.carry[t - 1] : 0ull;
     lds_barrier();
@@ -613,6 +623,33 @@ __device__ __forceinline__ void pow5(Smem<LOGM> &sm, const Twiddles &T, const Co
         tproduct<LOGM>(sm, T, K, x, 0, M / 2, nullptr, x, M, ysave);
         if ((e >> b) & 1) mul_small_vec<C>(x, 5u, sm.sc);
     }
+}
+
+// r <- sum of digits[i] 10^(13 i) over i < n (digits in LDS, each below 2^46).
+template <int C>
+__device__ __forceinline__ void from_digits(uint32_t (&r)[C], const uint64_t *digits, int n, Scratch &sc)
+{
+#pragma unroll
+    for (int i = 0; i < C; i++) r[i] = 0u;
+    for (int i = n - 1; i >= 0; i--) {          // 10^13 = 10^6 10^7
+        mul_small_vec<C>(r, 1000000u, sc);
+        mul_small_vec<C>(r, 10000000u, sc, digits[i]);
+    }
+}
+
+// The slot's canonical digits (left at scr by dec::launch_norm) as a number
+// below N.
+template <int LOGM>
+__device__ __forceinline__ void dec_value(Smem<LOGM> &sm, const Dev &D, int c, uint32_t (&r)[G<LOGM>::C])
+{
+    constexpr int C = G<LOGM>::C;
+    const int Lw = D.form[c].Lw;
+    const double *src = (const double *)(D.scr + (size_t)c * 2 * G<LOGM>::M);
+    uint64_t *dg = (uint64_t *)sm.X;
+    for (int i = threadIdx.x; i < Lw; i += THREADS) dg[i] = (uint64_t)src[i];
+    __syncthreads();
+    from_digits<C>(r, dg, Lw, sm.sc);
+    reduce_once<C>(r, D.N + (size_t)c * D.stride, D.Ls[c], 0, sm.sc);
 }
 
 // N = sum of coef * 10^exp over the candidate's terms; one workgroup each.
@@ -829,6 +866,41 @@ __global__ __launch_bounds__(THREADS) void setup_kernel(Dev D, Twiddles T, Const
     }
 }
 
+// dig (zeroed, Lw + 1 limbs) += base R mod N for R = 10^(D + f): base times
+// 10^f Q - q N = (10^f + q) Q - q 10^D, q = 10^f Q / N to 15 digits, so that
+// the value stays far below R.  Only the limbs around 10^D, where the two
+// cancel, need carries.  One thread.
+__device__ void dec_start(double *dig, const dec::Form &f, uint32_t base)
+{
+    typedef unsigned __int128 u128;
+    const u128 B = 10000000000000ull;
+    double ten = 1.0, rho = 0.0;
+    for (int i = 0; i < f.f; i++) ten *= 10.0;                  // exact: f <= 20
+    for (int k = 0; k < f.nt - 1; k++) {
+        double v = -f.t[k].c;
+        for (int e = dec::DIGITS * f.t[k].E + f.t[k].s; e < f.D && v > 1e-40; e++) v /= 10.0;
+        rho += v;                                               // Q / 10^D < 0.1
+    }
+    const u128 q = (u128)(ten * rho / (1.0 - rho)), tenf = (u128)ten;
+    for (int k = -1; k < f.nt; k++) {       // Q's 1, its terms, then -q 10^D
+        const bool last = k == f.nt - 1;
+        const int e = k < 0 ? 0 : dec::DIGITS * f.t[k].E + f.t[k].s;
+        u128 w = last ? q * base : (tenf + q) * base * (uint32_t)(k < 0 ? 1.0 : -f.t[k].c);
+        for (int i = 0; i < e % dec::DIGITS; i++) w *= 10u;
+        for (int E = e / dec::DIGITS; w; E++, w /= B) {
+            const double v = (double)(uint64_t)(w % B);
+            dig[E] += last ? -v : v;
+        }
+    }
+    double c = 0.0;
+    const int ED = f.D / dec::DIGITS;
+    for (int i = ED > 4 ? ED - 4 : 0; i <= f.Lw; i++) {
+        const double x = dig[i] + c;
+        c = __builtin_rint(x * dec::IB);
+        dig[i] = __builtin_fma(-c, dec::B, x);
+    }
+}
+
 // Start a round: r = base * R mod N, bitpos = nbits - 2 (the top bit of d
 // is 1 and is consumed by the initial value).
 // mode 0: every alive slot, with `base`.
@@ -872,6 +944,22 @@ __global__ __launch_bounds__(THREADS) void round_start_kernel(Dev D, uint32_t ba
         if (!D.alive[c] || D.pre[c]) return;
         if (threadIdx.x == 0) D.base[c] = base;
     }
+    if (D.form) {
+        const dec::Form &f = D.form[c];
+        const int lm = base <= (uint32_t)dec::MAX_BASE ? f.lm : 0;
+        if (threadIdx.x == 0) D.path[c] = lm;
+        if (lm) {       // base, or base R = base 10^f Q in Montgomery form
+            double *dig = D.dig + (size_t)c * D.dstride;
+            for (int i = threadIdx.x; i <= f.Lw; i += THREADS) dig[i] = 0.0;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                if (f.mode == dec::TOP) dig[0] = (double)base;
+                else dec_start(dig, f, base);
+                D.bitpos[c] = D.nbits[c] - 2;
+            }
+            return;
+        }
+    }
     const int L = D.Ls[c];
     uint32_t r[C];
     load_vec<C>(r, D.one + (size_t)c * D.stride, L, 0);
@@ -889,7 +977,7 @@ __global__ __launch_bounds__(THREADS) void exp_kernel(Dev D, Twiddles T, Consts 
     __shared__ Smem<LOGM> sm;
     const int c = slot_id(D);
     if (D.run && !D.run[c]) return;      // (slots under admission are not touched)
-    if (!D.alive[c] || D.pre[c]) return;
+    if (!D.alive[c] || D.pre[c] || (D.path && D.path[c])) return;
     const int s = D.sval[c];
     int bp = D.bitpos[c];
     if (bp < s) return;
@@ -948,6 +1036,25 @@ __global__ __launch_bounds__(THREADS) void round_end_kernel(Dev D, Twiddles T, C
     const uint32_t *one = D.one + (size_t)c * D.stride;
     const uint32_t *nm1 = D.nm1 + (size_t)c * D.stride;
     uint32_t r[C];
+    if (D.path && D.path[c]) {      // digits: plain residue, s = 1
+        dec_value<LOGM>(sm, D, c, r);
+        if (out) store_vec<C>(r, out + (size_t)c * out_stride, L, 0);
+        uint32_t n[C];
+        load_vec<C>(n, D.N + (size_t)c * D.stride, L, 0);
+        bool no1 = false, nom = false, no0 = false;
+#pragma unroll
+        for (int i = 0; i < C; i++) {
+            const uint32_t u = threadIdx.x == 0 && i == 0 ? 1u : 0u;
+            no1 |= r[i] != u;
+            nom |= r[i] != n[i] - u;                            // N is odd
+            no0 |= r[i] != 0u;
+        }
+        no1 = block_any(no1, sm.sc);
+        nom = block_any(nom, sm.sc);
+        no0 = block_any(no0, sm.sc);
+        if (threadIdx.x == 0 && no1 && nom && no0) D.alive[c] = 0;
+        return;
+    }
     load_vec<C>(r, D.res + (size_t)c * D.stride, L, L);
     bool pass = vec_equal_mem<C>(r, one, L, L, sm.sc) || vec_equal_mem<C>(r, nm1, L, L, sm.sc) ||
                 vec_equal_mem<C>(r, one, 0, L, sm.sc);          // r == 0: base == 0 (mod N)
@@ -1035,9 +1142,134 @@ __device__ __forceinline__ void store_vec64(const uint32_t (&v)[C], uint64_t *ds
     for (int idx = len + (int)threadIdx.x; idx < ld; idx += THREADS) dst[idx] = 0u;
 }
 
+// a <- R^2 mod N in the high layout, as 2^(24 L) in Montgomery form
+// (left-to-right powering of 2, squarings and doublings).
+template <int LOGM>
+__device__ __forceinline__ void mont_r2(Smem<LOGM> &sm, const Twiddles &T, const Consts &K, const Dev &D, int c,
+                                        uint32_t (&a)[G<LOGM>::C])
+{
+    constexpr int M = G<LOGM>::M, C = G<LOGM>::C;
+    const int L = D.Ls[c];
+    load_vec<C>(a, D.one + (size_t)c * D.stride, L, L);       // Montgomery form of 1
+    const uint32_t e = 24u * (uint32_t)L;
+    for (int i = 31 - __clz((int)e); i >= 0; i--) {
+        montmul<LOGM>(sm, T, K, D, c, a, L, nullptr);
+        if ((e >> i) & 1u)
+            mulsmall_modN<C>(a, 2u, D.N + (size_t)c * D.stride, L, L, sm.X, sm.sc,
+                             D.Nh + (size_t)c * M);
+    }
+}
+
+// Checkpoint: D.res <- the residue in progress in Montgomery form, from the
+// canonical digits dec::launch_norm left (slots on the digit path only).
+template <int LOGM>
+__global__ __launch_bounds__(THREADS) void dec_save_kernel(Dev D, Twiddles T, Consts K)
+{
+    constexpr int M = G<LOGM>::M, C = G<LOGM>::C;
+    __shared__ Smem<LOGM> sm;
+    const int c = slot_id(D);
+    if (!D.path[c] || D.pre[c]) return;
+    const int L = D.Ls[c];
+    uint32_t *res = D.res + (size_t)c * D.stride, *scr = D.scr + (size_t)c * 2 * M;
+    uint32_t r[C];
+    dec_value<LOGM>(sm, D, c, r);
+    store_vec<C>(r, res, L, 0);
+    __syncthreads();
+    mont_r2<LOGM>(sm, T, K, D, c, r);
+    store_vec<C>(r, scr, L, L);
+    __syncthreads();
+    load_vec<C>(r, scr, L, 0);
+    __syncthreads();
+    to_fft<LOGM>(sm, T, K, r, L, scr, D.ysv + (size_t)c * G<LOGM>::YSV + M);
+    load_vec<C>(r, res, L, 0);
+    montmul<LOGM>(sm, T, K, D, c, r, 0, scr);
+    store_vec<C>(r, res, L, L);
+}
+
+// Resume: digits of the Montgomery residue at D.res, for the slots info[3 i]
+// on the digit path: REDC(res), or res times base-10^13 Montgomery's R (10^f
+// Q), then base 2^24 to base 10^13 by Horner's rule over the limbs (balanced
+// digits, carries one limb per step).
+template <int LOGM>
+__global__ __launch_bounds__(THREADS) void dec_load_kernel(Dev D, Twiddles T, Consts K, const int32_t *info)
+{
+    constexpr int M = G<LOGM>::M, C = G<LOGM>::C;
+    constexpr int ND = (M * 3 / 10 + THREADS - 1) / THREADS;    // Lw < 0.28 M
+    __shared__ Smem<LOGM> sm;
+    const int c = info[3 * blockIdx.x];
+    if (!D.path[c] || D.pre[c]) return;
+    const dec::Form &f = D.form[c];
+    const int L = D.Ls[c], Lw = f.Lw, t = tid_();
+    const uint32_t *Nl = D.N + (size_t)c * D.stride;
+    uint32_t *scr = D.scr + (size_t)c * 2 * M;
+    uint32_t r[C];
+    if (f.mode == dec::TOP) {
+#pragma unroll
+        for (int i = 0; i < C; i++) r[i] = t == 0 && i == 0 ? 1u : 0u;
+    } else {
+        uint64_t *dg = (uint64_t *)sm.X;
+        for (int i = threadIdx.x; i < Lw; i += THREADS) dg[i] = 0ull;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            dg[0] = 1ull;
+            for (int k = 0; k < f.nt - 1; k++) {
+                const uint64_t w = (uint64_t)f.t[k].ts, b = 10000000000000ull / w;
+                const uint64_t v = (uint64_t)-f.t[k].c;
+                dg[f.t[k].E] += v % b * w;
+                if (v >= b) dg[f.t[k].E + 1] += v / b;
+            }
+        }
+        __syncthreads();
+        from_digits<C>(r, dg, Lw, sm.sc);
+    }
+    to_fft<LOGM>(sm, T, K, r, L, scr, D.ysv + (size_t)c * G<LOGM>::YSV + M);
+    load_vec<C>(r, D.res + (size_t)c * D.stride, L, 0);
+    montmul<LOGM>(sm, T, K, D, c, r, 0, scr);
+    if (f.mode != dec::TOP)
+        for (int e = f.f; e > 0; e -= 7) {
+            uint32_t w = 1;
+            for (int i = 0; i < 7 && i < e; i++) w *= 10u;
+            mulsmall_modN<C>(r, w, Nl, L, L, sm.X, sm.sc, D.Nh + (size_t)c * M);
+        }
+    store_vec<C>(r, scr, L, L);
+    __syncthreads();
+    float *car = (float *)sm.X;                 // [2][Lw + 1] carries, |q| <= 2^23
+    double x[ND];
+#pragma unroll
+    for (int n = 0; n < ND; n++) x[n] = 0.0;
+    for (int i = threadIdx.x; i < 2 * Lw + 2; i += THREADS) car[i] = 0.0f;
+    __syncthreads();
+    uint32_t limb = scr[L - 1];
+    for (int i = L - 1; i >= 0; i--) {
+        float *in = car + (i & 1) * (Lw + 1);
+        if (threadIdx.x == 0) in[0] = (float)limb;
+        limb = i ? scr[i - 1] : 0u;
+#pragma unroll
+        for (int n = 0; n < ND; n++) {
+            const int k = t + n * THREADS;
+            if (k < Lw) {
+                // (the top limb keeps its whole value: below B, maybe above B/2)
+                const double h = x[n] * 16777216.0, q = k + 1 < Lw ? __builtin_rint(h * dec::IB) : 0.0;
+                x[n] = __builtin_fma(-q, dec::B, h);
+                in[k + 1] = (float)q;
+            }
+        }
+        lds_barrier();
+#pragma unroll
+        for (int n = 0; n < ND; n++) {
+            const int k = t + n * THREADS;
+            if (k < Lw) x[n] += (double)in[k];
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < ND; n++) {
+        const int k = t + n * THREADS;
+        if (k < Lw) D.dig[(size_t)c * D.dstride + k] = x[n];
+    }
+}
+
 // op AR_MUL: out = A B R^-1 mod N; AR_SQ: A^2 R^-1; AR_CHECK: flag = (A ==
-// R mod N or A == (N-1) R mod N); AR_R2: r2 = R^2 mod N (as 2^(24 L) in
-// Montgomery form: left-to-right powering of 2, squarings and doublings);
+// R mod N or A == (N-1) R mod N); AR_R2: r2 = R^2 mod N;
 // AR_TORES: out = A R mod N (A < N, times r2); AR_FROMRES: out = A R^-1 mod
 // N.  Slots decided without rounds (even N, N < 4) get zeros and flag 0.
 template <int LOGM>
@@ -1073,14 +1305,7 @@ __global__ __launch_bounds__(THREADS) void arith_kernel(Dev D, Twiddles T, Const
         return;
     }
     if (op == AR_R2) {
-        const uint32_t *Nl = D.N + (size_t)c * D.stride;
-        load_vec<C>(a, D.one + (size_t)c * D.stride, L, L);   // Montgomery form of 1, high layout
-        const uint32_t e = 24u * (uint32_t)L;
-        for (int i = 31 - __clz((int)e); i >= 0; i--) {
-            montmul<LOGM>(sm, T, K, D, c, a, L, nullptr);
-            if ((e >> i) & 1u)
-                mulsmall_modN<C>(a, 2u, Nl, L, L, sm.X, sm.sc, D.Nh + (size_t)c * M);
-        }
+        mont_r2<LOGM>(sm, T, K, D, c, a);
         store_vec<C>(a, r2 + (size_t)c * D.stride, L, L);
         return;
     }
@@ -1232,6 +1457,10 @@ struct mr_ctx {
     Twiddles T{};
     std::vector<void *> allocs;
     std::vector<int32_t> sval;
+    // classes of the base-10^13 path its candidates run in (bit lm), and
+    // whether some take the Montgomery step (bit 0)
+    uint32_t classes = 1u;
+    const double *tab[dec::MAX_LM + 1] = {};
 };
 
 namespace {
@@ -1288,8 +1517,18 @@ void geometry(long bits, int min_logm, int *L_out, int *logm_out)
 // Upper bound on the bit length of a number of `digits` decimal digits.
 long digits_to_bits(int64_t digits) { return (long)((double)digits * 3.3219280948873623) + 2; }
 
-// Geometry and device arrays for numbers of at most `bits` bits.
-int ctx_alloc_all(mr_ctx *x, long bits, int min_logm)
+// Decimal limbs of a number of at most `bits` bits on the base-10^13 path.
+int dec_limbs(long bits) { return (int)((double)bits * 0.30102999566398120 + 1.0 + 8.0) / dec::DIGITS + 2; }
+
+dec::Args dec_args(const Dev &d, int logm)
+{
+    return dec::Args{d.list, d.run, d.form, d.path, d.dig, d.dstride, d.N, d.stride, d.bitpos, d.sval,
+                     d.alive, d.pre, d.base, d.scr, 2 << logm, d.decNt, d.park, d.tstride, d.pstride};
+}
+
+// Geometry and device arrays for numbers of at most `bits` bits; with_dec:
+// also the base-10^13 path's, dense_lm: up to which class with N' (0: none).
+int ctx_alloc_all(mr_ctx *x, long bits, int min_logm, bool with_dec = false, int dense_lm = 0)
 {
     int L, logm;
     geometry(bits, min_logm, &L, &logm);
@@ -1330,6 +1569,16 @@ int ctx_alloc_all(mr_ctx *x, long bits, int min_logm)
     MR_ALLOC(base, uint32_t, n);
     MR_ALLOC(bidx, int32_t, n);
     MR_ALLOC(done, uint8_t, n);
+    if (with_dec) {
+        d.dstride = dec_limbs(bits);
+        MR_ALLOC(form, dec::Form, n);
+        MR_ALLOC(path, int32_t, n);
+        MR_ALLOC(dig, double, n * d.dstride);
+        d.tstride = dense_lm ? 2 << dense_lm : 0;
+        MR_ALLOC(decNt, double, dense_lm ? n * d.tstride : 1);
+        d.pstride = 2 * d.dstride + (dec_limbs(bits) * 2 + 4 > 1 << 13 ? 3 << dec::MAX_LM >> 1 : 0);
+        MR_ALLOC(park, double, n * d.pstride);
+    }
 #undef MR_ALLOC
     d.list = nullptr;
     fill_i32_kernel<<<(x->n + 255) / 256, 256, 0, x->st>>>(d.Ls, x->n, L);
@@ -1475,6 +1724,28 @@ extern "C" int mr_ctx_moduli(const mr_ctx_t *x, uint32_t *out)
 
 namespace {
 
+// One chunk of squarings over the whole context: every class its candidates
+// run in, and the Montgomery step where some need it (all bases above
+// MAX_BASE do).
+int launch_steps(mr_ctx *x, uint32_t classes, int steps)
+{
+    const dec::Args A = dec_args(x->d, x->logm);
+    for (int lm = dec::MIN_LM; lm <= dec::MAX_LM; lm++)
+        if (classes >> lm & 1u) dec::launch_exp(lm, A, x->tab[lm], x->n, steps, x->st);
+    if (!(classes & 1u)) return 0;
+    return dispatch_logm(x->logm, [&](auto lg) {
+        exp_kernel<decltype(lg)::value><<<x->n, THREADS, 0, x->st>>>(x->d, x->T, x->K, steps);
+        return 0;
+    });
+}
+
+// The classes in use when a round's bases are at most max_base.
+uint32_t round_classes(const mr_ctx *x, uint32_t min_base, uint32_t max_base)
+{
+    if (min_base > (uint32_t)dec::MAX_BASE) return 1u;
+    return x->classes | (max_base > (uint32_t)dec::MAX_BASE ? 1u : 0u);
+}
+
 // Rounds of every base in order over the whole context.  all_bases = false:
 // a candidate retires at its first failing base (its later rounds are not
 // run); true: every base is run on every candidate, as the reference runner
@@ -1529,8 +1800,12 @@ int run_rounds(mr_ctx *x, const uint32_t *bases, int n_bases, bool all_bases,
                 round_start_kernel<LG><<<n, THREADS, 0, x->st>>>(x->d, 0u, 3, dbases, n);
             else
                 round_start_kernel<LG><<<n, THREADS, 0, x->st>>>(x->d, base, 0, nullptr, 0);
-            for (int done = 0; done < max_bits; done += CHUNK)
-                exp_kernel<LG><<<n, THREADS, 0, x->st>>>(x->d, x->T, x->K, CHUNK);
+            const uint32_t cls = per_slot
+                ? round_classes(x, *std::min_element(bases, bases + n), *std::max_element(bases, bases + n))
+                : round_classes(x, base, base);
+            for (int done = 0; done < max_bits; done += CHUNK) (void)launch_steps(x, cls, CHUNK);
+            for (int lm = dec::MIN_LM; lm <= dec::MAX_LM; lm++)
+                if (cls >> lm & 1u) dec::launch_norm(lm, dec_args(x->d, x->logm), n, x->st);
             if (residues_out) {
                 MR_CHECK(hipMemsetAsync(dlimbs, 0, sizeof(uint32_t) * (size_t)n * x->stride, x->st));
                 round_end_kernel<LG><<<n, THREADS, 0, x->st>>>(x->d, x->T, x->K, dlimbs, x->stride);
@@ -1908,6 +2183,17 @@ __host__ __device__ bool cand_terms(int64_t a, int64_t b, int64_t c, uint64_t k,
     return true;
 }
 
+// How a candidate of `digits` digits runs, from the exponents its sparse
+// terms can reach: k and j of nk and nj digits (their sum may carry one
+// further).
+dec::Choice dec_choice(int64_t a, int64_t b, int64_t c, int nk, int nj, int which, int64_t digits)
+{
+    const int64_t lo = std::min(b, c), hi = std::max(b + nk, c + nj);
+    if (which == 0) return dec::choose(digits, lo, hi + 1);
+    if (which == 1) return dec::choose(digits, digits - 1 - hi, digits - lo);
+    return dec::choose(digits, std::min(a - b - nk, a - c - nj), a - lo);
+}
+
 // Where an admitted job's terms come from: the host (list == nullptr, terms
 // copied with the admission) or entry idx of a device survivor list.
 struct SurvJob {
@@ -1955,6 +2241,8 @@ extern "C" mr_ctx_t *mr_ctx_create_sparse(const mr_candidate_t *cands, int n_bat
 {
     if (!cands || n_batch < 1) return nullptr;
     std::vector<int64_t> terms((size_t)n_batch * TMAX * 2, 0);
+    std::vector<int32_t> choice((size_t)n_batch * 3, 0);
+    uint32_t classes = 0, dense = 0;        // bit lm
     int64_t max_digits = 1;
     for (int i = 0; i < n_batch; i++) {
         std::vector<std::pair<int64_t, int64_t>> t;
@@ -1970,11 +2258,26 @@ extern "C" mr_ctx_t *mr_ctx_create_sparse(const mr_candidate_t *cands, int n_bat
             terms[((size_t)i * TMAX + q) * 2 + 1] = t[q].second;
         }
         if (dg > max_digits) max_digits = dg;
+        const mr_candidate_t &cd = cands[i];
+        const dec::Choice ch = g_min_logm > MIN_LOGM ? dec::Choice{0, 0}
+            : dec_choice(cd.a, cd.b, cd.c, ndig_u(cd.k), ndig_u(cd.j), cd.which, dg);
+        choice[3 * (size_t)i] = (int32_t)dg;
+        choice[3 * (size_t)i + 1] = ch.lm;
+        choice[3 * (size_t)i + 2] = ch.mode;
+        classes |= 1u << ch.lm;
+        if (ch.lm && ch.mode == dec::DENSE) dense |= 1u << ch.lm;
     }
     const long bits = digits_to_bits(max_digits);
     mr_ctx *x = ctx_new((int)((bits + 31) / 32), n_batch, device);
     if (!x) return nullptr;
-    int rc = ctx_alloc_all(x, (long)x->n_words * 32, g_min_logm);
+    int rc = ctx_alloc_all(x, (long)x->n_words * 32, g_min_logm, true, dense ? 31 - __builtin_clz(dense) : 0);
+    x->classes = classes;
+    for (int lm = dec::MIN_LM; lm <= dec::MAX_LM && rc == 0; lm++)
+        if (classes >> lm & 1u && !(x->tab[lm] = dec::tables(x->device, lm))) rc = -2;
+    int32_t *dchoice = nullptr;
+    if (rc == 0 && ctx_alloc(x, (void **)&dchoice, sizeof(int32_t) * choice.size()) != 0) rc = -2;
+    if (rc == 0 && hipMemcpyAsync(dchoice, choice.data(), sizeof(int32_t) * choice.size(),
+                                  hipMemcpyHostToDevice, x->st) != hipSuccess) rc = -2;
     int64_t *dterms = nullptr;
     if (rc == 0 && ctx_alloc(x, (void **)&dterms, sizeof(int64_t) * terms.size()) != 0) rc = -2;
     if (rc == 0 && hipMemcpyAsync(dterms, terms.data(), sizeof(int64_t) * terms.size(),
@@ -1982,6 +2285,9 @@ extern "C" mr_ctx_t *mr_ctx_create_sparse(const mr_candidate_t *cands, int n_bat
     if (rc == 0)
         rc = dispatch_logm(x->logm, [&](auto lg) {
             constexpr int LG = decltype(lg)::value;
+            dec::launch_form(nullptr, x->n, dterms, TMAX, dchoice, x->d.form, x->d.err, x->st);
+            for (int lm = dec::MIN_LM; lm <= dec::MAX_LM; lm++)
+                if (dense >> lm & 1u) dec::launch_prepare(lm, dec_args(x->d, x->logm), x->tab[lm], x->n, x->st);
             build_kernel<LG><<<x->n, THREADS, 0, x->st>>>(x->d, x->T, x->K, dterms, TMAX, nullptr);
             return 0;
         });
@@ -2016,7 +2322,7 @@ extern "C" int mr_time_squarings(mr_ctx_t *x, uint32_t base, int n_bits, float *
         const int CHUNK = 256;
         for (int done = 0; done < n_bits; done += CHUNK) {
             const int steps = n_bits - done < CHUNK ? n_bits - done : CHUNK;
-            exp_kernel<LG><<<n, THREADS, 0, x->st>>>(x->d, x->T, x->K, steps);
+            (void)launch_steps(x, round_classes(x, base, base), steps);
         }
         (void)hipEventRecord(e1, x->st);
         return 0;
@@ -2056,6 +2362,7 @@ struct Req {
     double t_submit, t_admit;
     int L, logm;
     int64_t digits = 0;             // decimal length (sets L and logm)
+    dec::Choice choice = {0, 0};    // class and mode of its squarings
     int rounds;
     int64_t terms[TMAX * 2];
     // restored from a checkpoint after admission: the base in progress, the
@@ -2070,12 +2377,25 @@ struct Req {
 };
 
 
+// Numbers a pool holds: up to (2^logm - 2) / 2 limbs, the transform length's.
+long pool_bits(int logm) { return 24l * std::min<long>(((1l << logm) - 2) / 2, MAX_LIMBS) - 1; }
+
+// The largest base-10^13 class of a pool's numbers.
+int dec_pool_lm(int logm)
+{
+    int lm = dec::MIN_LM;
+    while (lm < dec::MAX_LM && (1 << lm) < 2 * dec_limbs(pool_bits(logm)) + 4) lm++;
+    return lm;
+}
+
 // Bytes of device memory per slot of a pool of transform length 2^logm
 // (the arrays of ctx_alloc_all).
 int64_t slot_bytes(int logm)
 {
     const int64_t M = 1ll << logm;
-    return 4 * (4 * M + 7 * M + (split_logm(logm) ? M + M / 2 : 0) + (half_logm(logm) ? M : 0)) + 32;
+    return 4 * (4 * M + 7 * M + (split_logm(logm) ? M + M / 2 : 0) + (half_logm(logm) ? M : 0)) + 32 +
+           (int64_t)sizeof(dec::Form) + 4 + 24 * dec_limbs(pool_bits(logm)) + 16 * (1ll << dec_pool_lm(logm)) +
+           (dec_pool_lm(logm) > 13 ? 12ll << dec::MAX_LM : 0);
 }
 
 struct Pool {
@@ -2090,8 +2410,13 @@ struct Pool {
     int32_t *d_resume = nullptr;    // [n][3] slot, base index, exponent bit
     uint8_t *d_run = nullptr;       // [n] slots that square in the next chunk
     uint8_t *h_run = nullptr;
-    hipGraph_t graph = nullptr;     // one chunk: run flags in, squarings, exponent bits out
-    hipGraphExec_t gexec = nullptr;
+    // one chunk (run flags in, squarings, exponent bits out) as a graph, per
+    // set of classes that occurred among the running slots
+    struct Chunk { uint32_t classes; hipGraph_t g; hipGraphExec_t ge; };
+    std::vector<Chunk> graphs;
+    hipStream_t st_cls[dec::MAX_LM + 1] = {};   // the classes' branches
+    hipEvent_t ev_fork = nullptr, ev_cls[dec::MAX_LM + 1] = {};
+    int32_t *h_choice = nullptr, *d_choice = nullptr;  // [n][3] digits, class, mode
     int32_t *h_resume = nullptr;
     uint32_t *h_resres = nullptr;   // [n][stride] residues to resume (pinned, on first use)
     // pinned host mirrors
@@ -2145,13 +2470,21 @@ void pool_free(Pool *p)
     if (!p) return;
     if (p->st_run) (void)hipStreamSynchronize(p->st_run);
     if (p->x && p->x->st) (void)hipStreamSynchronize(p->x->st);
-    if (p->gexec) (void)hipGraphExecDestroy(p->gexec);
-    if (p->graph) (void)hipGraphDestroy(p->graph);
+    for (Pool::Chunk &g : p->graphs) {
+        (void)hipGraphExecDestroy(g.ge);
+        (void)hipGraphDestroy(g.g);
+    }
+    for (int lm = 0; lm <= dec::MAX_LM; lm++) {
+        if (p->st_cls[lm]) (void)hipStreamDestroy(p->st_cls[lm]);
+        if (p->ev_cls[lm]) (void)hipEventDestroy(p->ev_cls[lm]);
+    }
+    if (p->ev_fork) (void)hipEventDestroy(p->ev_fork);
     if (p->ev_run) (void)hipEventDestroy(p->ev_run);
     if (p->ev_adm) (void)hipEventDestroy(p->ev_adm);
     if (p->st_run) (void)hipStreamDestroy(p->st_run);
     void *hp[] = {p->h_list_adm, p->h_Ls, p->h_bitpos, p->h_sval, p->h_terms, p->h_sjobs,
-                  p->h_alive, p->h_done, p->h_err, p->h_resume, p->h_resres, p->h_run};
+                  p->h_alive, p->h_done, p->h_err, p->h_resume, p->h_resres, p->h_run,
+                  p->h_choice};
     for (void *q : hp) if (q) (void)hipHostFree(q);
     if (p->x) mr_ctx_destroy(p->x);       // frees the device arrays it owns
     delete p;
@@ -2171,10 +2504,7 @@ int pool_new(mr_sched *S, int logm, Pool **out)
     p->chunk = S->bucket_chunk[logm] ? S->bucket_chunk[logm] : S->chunk;
     p->x = ctx_new(1, n, S->device);
     int rc = p->x ? 0 : -2;
-    // numbers of up to (2^logm - 2) / 2 limbs (24 lmax - 1 bits): the pool's
-    // transform length
-    const long lmax = std::min<long>(((1l << logm) - 2) / 2, MAX_LIMBS);
-    if (rc == 0) rc = ctx_alloc_all(p->x, 24l * lmax - 1, logm);
+    if (rc == 0) rc = ctx_alloc_all(p->x, pool_bits(logm), logm, true, dec_pool_lm(logm));
     if (rc == 0 && p->x->logm != logm) rc = -1;
     auto dev = [&](void **q, size_t b) { if (rc == 0 && ctx_alloc(p->x, q, b) != 0) rc = -2; };
     dev((void **)&p->d_list_adm, 4 * (size_t)n);
@@ -2184,6 +2514,7 @@ int pool_new(mr_sched *S, int logm, Pool **out)
     dev((void **)&p->d_bases, 4 * (size_t)S->n_bases);
     dev((void **)&p->d_resume, 12 * (size_t)n);
     dev((void **)&p->d_run, (size_t)n);
+    dev((void **)&p->d_choice, 12 * (size_t)n);
     auto host = [&](void **q, size_t b) {
         if (rc == 0 && hipHostMalloc(q, b ? b : 4, hipHostMallocDefault) != hipSuccess) rc = -2;
     };
@@ -2198,6 +2529,7 @@ int pool_new(mr_sched *S, int logm, Pool **out)
     host((void **)&p->h_err, 4);
     host((void **)&p->h_resume, 12 * (size_t)n);
     host((void **)&p->h_run, (size_t)n);
+    host((void **)&p->h_choice, 12 * (size_t)n);
     if (rc == 0 && (hipStreamCreateWithFlags(&p->st_run, hipStreamNonBlocking) != hipSuccess ||
                     hipEventCreateWithFlags(&p->ev_run, hipEventDisableTiming) != hipSuccess ||
                     hipEventCreateWithFlags(&p->ev_adm, hipEventDisableTiming) != hipSuccess))
@@ -2265,35 +2597,61 @@ void finish(mr_sched *S, int r, int verdict)
     S->n_done++;
 }
 
-// The pool's chunk as a HIP graph, captured once: copy the run flags in,
-// one squaring kernel over every slot of the pool (slots not running return
-// at once), copy the exponent bits out.  Fixed pointers and chunk length,
-// so each chunk is one hipGraphLaunch; no memset nodes.
-int pool_graph(mr_sched *S, Pool *p)
+// The pool's chunk over slots of the given classes as a HIP graph, captured
+// once per set of classes: copy the run flags in, one kernel per class over
+// every slot of the pool (slots of another class, or not running, return at
+// once), the classes side by side on branches of their own, copy the exponent
+// bits out.  Fixed pointers and chunk length, so each chunk is one
+// hipGraphLaunch; no memset nodes.
+int pool_graph(Pool *p, uint32_t classes, hipGraphExec_t *out)
 {
+    for (const Pool::Chunk &g : p->graphs)
+        if (g.classes == classes) { *out = g.ge; return 0; }
     hipStream_t st = p->st_run;
     Dev Dg = p->x->d;
     Dg.list = nullptr;
     Dg.run = p->d_run;
     const int chunk = p->chunk, n = p->n;
-    MR_CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    hipError_t e = hipMemcpyAsync(p->d_run, p->h_run, (size_t)n, hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) {
+    const dec::Args A = dec_args(Dg, p->logm);
+    int first = 0;                       // the class that stays on the run stream
+    while (!(classes >> first & 1u)) first++;
+    for (int lm = first + 1; lm <= dec::MAX_LM; lm++) {
+        if (!(classes >> lm & 1u)) continue;
+        if (!p->ev_fork) MR_CHECK(hipEventCreateWithFlags(&p->ev_fork, hipEventDisableTiming));
+        if (!p->st_cls[lm]) MR_CHECK(hipStreamCreateWithFlags(&p->st_cls[lm], hipStreamNonBlocking));
+        if (!p->ev_cls[lm]) MR_CHECK(hipEventCreateWithFlags(&p->ev_cls[lm], hipEventDisableTiming));
+    }
+    const double *tab[dec::MAX_LM + 1] = {};
+    for (int lm = dec::MIN_LM; lm <= dec::MAX_LM; lm++)
+        if (classes >> lm & 1u && !(tab[lm] = dec::tables(p->x->device, lm))) return hip_fail(hipErrorOutOfMemory, "tables");
+    auto steps = [&](int lm, hipStream_t on) {
+        if (lm) { dec::launch_exp(lm, A, tab[lm], n, chunk, on); return; }
         (void)dispatch_logm(p->logm, [&](auto lg) {
             constexpr int LG = decltype(lg)::value;
-            exp_kernel<LG><<<n, THREADS, 0, st>>>(Dg, p->x->T, p->x->K, chunk);
+            exp_kernel<LG><<<n, THREADS, 0, on>>>(Dg, p->x->T, p->x->K, chunk);
             return 0;
         });
-        e = hipGetLastError();
+    };
+    MR_CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+    hipError_t e = hipMemcpyAsync(p->d_run, p->h_run, (size_t)n, hipMemcpyHostToDevice, st);
+    if (e == hipSuccess && p->ev_fork) e = hipEventRecord(p->ev_fork, st);
+    for (int lm = dec::MAX_LM; lm > first && e == hipSuccess; lm--) {     // longest first
+        if (!(classes >> lm & 1u)) continue;
+        e = hipStreamWaitEvent(p->st_cls[lm], p->ev_fork, 0);
+        if (e == hipSuccess) { steps(lm, p->st_cls[lm]); e = hipEventRecord(p->ev_cls[lm], p->st_cls[lm]); }
     }
+    if (e == hipSuccess) { steps(first, st); e = hipGetLastError(); }
+    for (int lm = first + 1; lm <= dec::MAX_LM && e == hipSuccess; lm++)
+        if (classes >> lm & 1u) e = hipStreamWaitEvent(st, p->ev_cls[lm], 0);
     if (e == hipSuccess)
         e = hipMemcpyAsync(p->h_bitpos, p->x->d.bitpos, 4 * (size_t)n, hipMemcpyDeviceToHost, st);
-    hipGraph_t g = nullptr;
-    const hipError_t e2 = hipStreamEndCapture(st, &g);
+    Pool::Chunk c = {classes, nullptr, nullptr};
+    const hipError_t e2 = hipStreamEndCapture(st, &c.g);
     if (e == hipSuccess) e = e2;
-    if (e == hipSuccess) e = hipGraphInstantiate(&p->gexec, g, nullptr, nullptr, 0);
-    p->graph = g;
-    if (e != hipSuccess) { p->gexec = nullptr; return hip_fail(e, "chunk graph"); }
+    if (e == hipSuccess) e = hipGraphInstantiate(&c.ge, c.g, nullptr, nullptr, 0);
+    if (e != hipSuccess) return hip_fail(e, "chunk graph");
+    p->graphs.push_back(c);
+    *out = c.ge;
     return 0;
 }
 
@@ -2301,15 +2659,19 @@ int pool_graph(mr_sched *S, Pool *p)
 int launch_chunk(mr_sched *S, Pool *p)
 {
     p->run_list.clear();
+    uint32_t classes = 0;
     for (int c = 0; c < p->n; c++) {
         const bool run = p->state[c] == SL_RUN;
         p->h_run[c] = run ? 1 : 0;
-        if (run) p->run_list.push_back(c);
+        if (!run) continue;
+        p->run_list.push_back(c);
+        classes |= 1u << S->reqs[p->req[c]].choice.lm;
     }
     if (p->run_list.empty()) return 0;
     const int nr = (int)p->run_list.size();
-    if (!p->gexec) { int rc = pool_graph(S, p); if (rc) return rc; }
-    MR_CHECK(hipGraphLaunch(p->gexec, p->st_run));
+    hipGraphExec_t ge = nullptr;
+    { int rc = pool_graph(p, classes, &ge); if (rc) return rc; }
+    MR_CHECK(hipGraphLaunch(ge, p->st_run));
     MR_CHECK(hipEventRecord(p->ev_run, p->st_run));
     const int chunk = p->chunk;
     p->run_busy = true;
@@ -2330,11 +2692,16 @@ void chunk_done(Pool *p)
 int launch_admin(mr_sched *S, Pool *p)
 {
     p->adm_list.clear();
+    uint32_t end_classes = 0;
     for (int c = 0; c < p->n; c++)
-        if (p->state[c] == SL_END) p->adm_list.push_back(c);
+        if (p->state[c] == SL_END) {
+            p->adm_list.push_back(c);
+            end_classes |= 1u << S->reqs[p->req[c]].choice.lm;
+        }
     const int n_end = (int)p->adm_list.size();
     int n_res = 0;          // restored candidates among the admitted
     int n_dev = 0;          // admitted from device survivor lists
+    uint32_t dense = 0;     // classes with N' to prepare
     std::vector<int> &queue = S->queue[p->logm];
     size_t &qh = S->qhead[p->logm];
     const int64_t per = slot_bytes(p->logm);
@@ -2351,6 +2718,10 @@ int launch_admin(mr_sched *S, Pool *p)
                                 q.cand.which};
         n_dev += q.dev_list ? 1 : 0;
         p->h_Ls[i] = q.L;
+        p->h_choice[3 * i] = (int32_t)q.digits;
+        p->h_choice[3 * i + 1] = q.choice.lm;
+        p->h_choice[3 * i + 2] = q.choice.mode;
+        if (q.choice.lm && q.choice.mode == dec::DENSE) dense |= 1u << q.choice.lm;
         if (q.resume_bidx >= 0) {
             if (!p->h_resres &&
                 hipHostMalloc(&p->h_resres, 4 * (size_t)p->n * p->x->stride, hipHostMallocDefault) != hipSuccess) {
@@ -2390,6 +2761,17 @@ int launch_admin(mr_sched *S, Pool *p)
                                                                  p->x->d.err);
             MR_CHECK(hipGetLastError());
         }
+        MR_CHECK(hipMemcpyAsync(p->d_choice, p->h_choice, 12 * (size_t)n_new, hipMemcpyHostToDevice, st));
+        dec::launch_form(p->d_list_adm + n_end, n_new, p->d_terms, TMAX, p->d_choice, p->x->d.form,
+                         p->x->d.err, st);
+        Dev Dp = p->x->d;
+        Dp.list = p->d_list_adm + n_end;
+        for (int lm = dec::MIN_LM; lm <= dec::MAX_LM; lm++) {
+            if (!(dense >> lm & 1u)) continue;
+            const double *tab = dec::tables(p->x->device, lm);
+            if (!tab) return hip_fail(hipErrorOutOfMemory, "tables");
+            dec::launch_prepare(lm, dec_args(Dp, p->logm), tab, n_new, st);
+        }
     }
     Dev De = p->x->d, Dn = p->x->d;
     De.list = p->d_list_adm;
@@ -2401,6 +2783,8 @@ int launch_admin(mr_sched *S, Pool *p)
     int rc = dispatch_logm(p->logm, [&](auto lg) {
         constexpr int LG = decltype(lg)::value;
         if (n_end) {
+            for (int lm = dec::MIN_LM; lm <= dec::MAX_LM; lm++)
+                if (end_classes >> lm & 1u) dec::launch_norm(lm, dec_args(De, p->logm), n_end, st);
             round_end_kernel<LG><<<n_end, THREADS, 0, st>>>(De, T, K, nullptr, 0);
             round_start_kernel<LG><<<n_end, THREADS, 0, st>>>(De, 0u, 2, bases, nb);
         }
@@ -2422,6 +2806,10 @@ int launch_admin(mr_sched *S, Pool *p)
         }
         MR_CHECK(hipMemcpyAsync(p->d_resume, p->h_resume, 12 * (size_t)n_res, hipMemcpyHostToDevice, st));
         resume_kernel<<<(n_res + 63) / 64, 64, 0, st>>>(p->x->d, p->d_resume, n_res, bases);
+        (void)dispatch_logm(p->logm, [&](auto lg) {
+            dec_load_kernel<decltype(lg)::value><<<n_res, THREADS, 0, st>>>(p->x->d, T, K, p->d_resume);
+            return 0;
+        });
         MR_CHECK(hipGetLastError());
     }
     const size_t n = (size_t)p->n;
@@ -2509,6 +2897,7 @@ bool make_req(const mr_candidate_t &cd, int64_t tag, Req &q)
     }
     geometry(digits_to_bits(dg), MIN_LOGM, &q.L, &q.logm);
     q.digits = dg;
+    q.choice = dec_choice(cd.a, cd.b, cd.c, ndig_u(cd.k), ndig_u(cd.j), cd.which, dg);
     if (q.logm > MAX_LOGM || q.L > MAX_LIMBS) {
         fprintf(stderr, "%s: candidate of %lld digits is beyond this build's transform sizes\n", kWho,
                 (long long)dg);
@@ -2540,7 +2929,9 @@ int enqueue(mr_sched *S, std::vector<Req> &add)
                     (long long)S->budget);
             return -1;
         }
+    const bool big = *std::max_element(S->bases.begin(), S->bases.end()) > (uint32_t)dec::MAX_BASE;
     for (Req &q : add) {
+        if (big) q.choice = dec::Choice{0, 0};      // a base too large for the digits' carry step
         q.t_submit = now;
         S->queue[q.logm].push_back((int)S->reqs.size());
         S->reqs.push_back(std::move(q));
@@ -2591,6 +2982,7 @@ int submit_survivors(mr_sched *S, long long a, long long b, long long c, const u
     // decimal digits, and one representative fixes the slot size
     Req proto;
     if (!make_req(mr_candidate_t{a, b, c, 1u, 1u, which}, 0, proto)) return -1;
+    proto.choice = dec_choice(a, b, c, 5, 5, which, proto.digits);
     for (uint32_t i = 0; i < n; i++) {
         Req &q = add[i];
         q = proto;
@@ -2648,6 +3040,28 @@ int sched_checkpoint(mr_sched *S, const char *path)
         std::vector<int32_t> bidx((size_t)p->n), bitpos((size_t)p->n);
         MR_CHECK(hipMemcpy(bidx.data(), p->x->d.bidx, 4 * (size_t)p->n, hipMemcpyDeviceToHost));
         MR_CHECK(hipMemcpy(bitpos.data(), p->x->d.bitpos, 4 * (size_t)p->n, hipMemcpyDeviceToHost));
+        // digits -> Montgomery residues of the slots on the base-10^13 path
+        int nd = 0;
+        uint32_t classes = 0;
+        for (int c = 0; c < p->n; c++) {
+            if (p->state[c] != SL_RUN && p->state[c] != SL_END) continue;
+            const int lm = S->reqs[p->req[c]].choice.lm;
+            if (lm) { p->h_list_adm[nd++] = c; classes |= 1u << lm; }
+        }
+        if (nd) {
+            hipStream_t st = p->x->st;
+            Dev D = p->x->d;
+            D.list = p->d_list_adm;
+            MR_CHECK(hipMemcpyAsync(p->d_list_adm, p->h_list_adm, 4 * (size_t)nd, hipMemcpyHostToDevice, st));
+            for (int lm = dec::MIN_LM; lm <= dec::MAX_LM; lm++)
+                if (classes >> lm & 1u) dec::launch_norm(lm, dec_args(D, p->logm), nd, st);
+            (void)dispatch_logm(p->logm, [&](auto lg) {
+                dec_save_kernel<decltype(lg)::value><<<nd, THREADS, 0, st>>>(D, p->x->T, p->x->K);
+                return 0;
+            });
+            MR_CHECK(hipGetLastError());
+            MR_CHECK(hipStreamSynchronize(st));
+        }
         for (int c = 0; c < p->n; c++) {
             if (p->state[c] != SL_RUN && p->state[c] != SL_END) continue;
             Row w{p->req[c], bidx[c], bitpos[c], {}};

@@ -1,0 +1,59 @@
+"""Base-10^13 rounds of search-form candidates on the GPU against GMP: residues
+a^d mod N at the digit counts where the transform class changes (13 (M/2 - 2)
+digits, less 8 in the Montgomery modes), with bases at the limit of the digits'
+carry step (511) and beyond it (512: the Montgomery step), and candidates that
+have to take the Montgomery step (no gap, or terms below 10^2)."""
+import pytest
+
+from _support import gmp_build, gmp_sprp
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("digits", [40, 312, 798, 799, 806, 807, 1630, 1639, 3302, 3303, 6622,
+                                    6631, 13286, 13287])
+def test_residues_at_class_edges(gpu, digits):
+    a = digits
+    cands = [(a, a // 2, 20, 4096, 4095, 0), (a, a // 2, 20, 4096, 4095, 1),
+             (a, a // 2 + 3, 15, 1, 999999, 2), (a, a - a // 10 - 7, a // 3, 77, 4096, 0),
+             (a, a - 1 - len("4096"), 3, 4096, 9, 0), (a, a // 2, 1, 5, 3, 0),
+             (a, a - a // 40 - 6, a // 20 + 3, 4096, 4095, 0), (a, a - a // 40 - 6, 3, 9, 4095, 1)]
+    bases = [2, 511, 512]
+    if digits > 4000:               # GMP's share of the time
+        cands, bases = cands[:2] + cands[-2:], [2]
+    ctx = gpu.MrContext(candidates=cands)
+    _, res, passed = ctx.run(bases, all_bases=True, passes=True)
+    for i, cd in enumerate(cands):
+        n = gmp_build(*cd)
+        for j, base in enumerate(bases):
+            ok, r, _ = gmp_sprp(n, base)
+            assert res[i][j] == r, (cd, base)
+            assert passed[i][j] == ok, (cd, base)
+    ctx.close()
+
+
+@pytest.mark.parametrize("digits", [26598, 26599])
+def test_residues_long(gpu, digits):
+    """Against the Montgomery step on the same numbers given as words."""
+    cands = [(digits, 20000, 9000, 4096, 4095, 0), (digits, 20000, 100, 77, 4095, 1),
+             (digits, 26000, 300, 4096, 4095, 0)]
+    ctx = gpu.MrContext(candidates=cands)
+    _, res = ctx.run([3])
+    ctx.close()
+    ref = gpu.MrContext([gmp_build(*cd) for cd in cands])
+    assert ref.run([3])[1] == res
+    ref.close()
+
+
+def test_classes_side_by_side_and_mixed_bases(gpu):
+    """One context over four classes and the Montgomery step, every slot with
+    its own base on either side of 511."""
+    cands = [(a, a // 2, 20 if i % 3 else 1, 4000 + i, 77, i & 1)
+             for i, a in enumerate([300, 900, 2000, 4000, 310, 1000, 2100, 3900])]
+    bases = [2, 3, 511, 512, 600, 7, 510, 65537]
+    ctx = gpu.MrContext(candidates=cands)
+    ok, res = ctx.run_per_slot(bases)
+    for cd, b, o, r in zip(cands, bases, ok, res):
+        want, wr, _ = gmp_sprp(gmp_build(*cd), b)
+        assert r == wr and o == bool(want), (cd, b)
+    ctx.close()

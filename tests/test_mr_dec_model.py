@@ -1,0 +1,116 @@
+"""CPU model of the base-10^13 squaring (mr_dec_core.h compiled for the host,
+one thread per lane): mul x^2 modulo N (times R^-1 in the BOTTOM mode) equals
+Python's integers, at the edges of every transform class, in both modes, from
+one fold round to the most, on random digits and on digits all of the largest
+magnitude (the longest sums and every tie of the carries)."""
+import ctypes as C
+import random
+import subprocess
+import sys
+
+import pytest
+
+from _support import ROOT
+
+if hasattr(sys, "set_int_max_str_digits"):
+    sys.set_int_max_str_digits(0)
+
+B = 10 ** 13
+TOP, BOTTOM, DENSE = 0, 1, 2
+
+
+@pytest.fixture(scope="module")
+def model(tmp_path_factory):
+    out = tmp_path_factory.mktemp("decmodel") / "mr_dec_model.so"
+    subprocess.run(["g++", "-O2", "-std=c++20", "-march=native", "-ffp-contract=off", "-shared",
+                    "-fPIC", "-pthread", f"-I{ROOT / 'prime-finder_amd' / 'csrc'}",
+                    str(ROOT / "tests" / "model" / "mr_dec_model.cpp"), "-o", str(out)],
+                   check=True)
+    L = C.CDLL(str(out))
+    L.dec_choose.argtypes = [C.c_longlong, C.c_longlong, C.c_longlong, C.POINTER(C.c_int)]
+    L.dec_square.argtypes = [C.POINTER(C.c_longlong), C.c_int, C.c_longlong, C.c_int, C.c_int,
+                             C.POINTER(C.c_double), C.POINTER(C.c_double), C.c_int]
+    return L
+
+
+def terms_of(D, b, c, k, j, rev):
+    """(coef, exp) pairs of N (or its decimal reversal) and the range of the
+    exponents below D."""
+    s = str(k * 10 ** b + j * 10 ** c)[::-1]
+    pos = [i for i, d in enumerate(s) if d != "0"]
+    e = [(D - 1 - i if rev else i) for i in pos]
+    return [(1, D), (-1, 0)] + [(-int(s[i]), x) for i, x in zip(pos, e)], min(e), max(e) + 1
+
+
+CASES = [
+    # D, b, c, k, j, rev, steps: class edges are 13 (M/2 - 2) digits
+    (300, 150, 40, 1234, 77, False, 3), (300, 150, 40, 1234, 77, True, 3),
+    (806, 700, 60, 9999, 9999, False, 2), (798, 700, 60, 999, 1, True, 3),
+    (807, 700, 60, 999, 1, False, 2), (1638, 1500, 60, 1000000, 999999, False, 2),
+    (1639, 1500, 60, 4096, 4096, True, 2), (3302, 1000, 100, 77, 5, False, 2),
+    (3303, 1000, 100, 77, 5, True, 2), (2695, 2663, 2002, 4096, 1, False, 1),
+    (6630, 3000, 2999, 4096, 4095, False, 1), (6631, 3000, 100, 4096, 4095, True, 1),
+    (13286, 9000, 5000, 4096, 4095, False, 1), (13287, 9000, 100, 2, 3, True, 1),
+    # DENSE: small gaps at both ends
+    (797, 760, 30, 9999, 9999, False, 2), (798, 760, 30, 999, 7, True, 2),
+    (1636, 1600, 90, 4096, 4095, True, 2), (3300, 3100, 100, 77, 4096, False, 2),
+    (6600, 6500, 200, 1000000, 999999, True, 1), (13000, 12500, 100, 4096, 4095, False, 1),
+    (26598, 9000, 5000, 4096, 4095, False, 1), (53000, 30000, 100, 4096, 4095, True, 1),
+    (100000, 49000, 100, 4096, 4095, True, 1),
+]
+
+
+@pytest.mark.parametrize("kind", ["random", "largest", "ends"])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}-{c[1]}-{c[2]}{'r' if c[5] else ''}")
+def test_square_step(model, case, kind):
+    D, b, c, k, j, rev, steps = case
+    if D > 14000 and kind == "ends":
+        pytest.skip("long host run; the shorter classes cover the pattern")
+    rng = random.Random(D * 7 + len(kind))
+    terms, lo, hi = terms_of(D, b, c, k, j, rev)
+    N = sum(q * 10 ** e for q, e in terms)
+    mode = C.c_int()
+    lm = model.dec_choose(D, lo, hi, C.byref(mode))
+    assert lm >= 7
+    if D in (797, 798, 1636, 3300, 6600, 13000):
+        assert mode.value == DENSE
+    Lw = (D + (0 if mode.value == TOP else 8) + 12) // 13
+    assert 2 * Lw + 4 <= 1 << lm and (lm == 7 or 2 * Lw + 6 > 1 << (lm - 1))
+    dig = (C.c_double * Lw)()
+    for i in range(Lw):
+        dig[i] = {"random": rng.randint(-B // 2, B // 2), "largest": B // 2,
+                  "ends": rng.choice([-1, 1]) * (B // 2)}[kind]
+    if mode.value != TOP:
+        dig[Lw - 1] = 0
+    x = sum(int(dig[i]) * B ** i for i in range(Lw))
+    muls = [rng.choice([1, 2, 7, 511]) for _ in range(steps)]
+    flat = [v for t in terms for v in t]
+    got = model.dec_square((C.c_longlong * len(flat))(*flat), len(terms), D, lm, mode.value, dig,
+                           (C.c_double * steps)(*muls), steps)
+    assert got == Lw
+    y = sum(int(dig[i]) * B ** i for i in range(Lw))
+    if mode.value == TOP:
+        mod = N * 10 ** (13 * Lw - D)
+        for m in muls:
+            x = x * x * m % mod
+        assert (x - y) % mod == 0
+    else:           # y R^(2^steps - 1) = x^(2^steps) prod mul^(2^(steps - 1 - i)), no inverse needed
+        z = x
+        for m in muls:
+            z = z * z * m % N
+        assert (y * pow(B ** Lw % N, 2 ** steps - 1, N) - z) % N == 0
+    assert max(abs(v) for v in dig) <= B / 2 + 2 ** 16
+    assert 10 * abs(y) <= 6 * (B ** Lw if mode.value == TOP else N)
+
+
+def test_what_is_not_taken(model):
+    """Short numbers, terms that leave no gap, and a least exponent below 2
+    (N - 1 may be divisible by 4) stay with the Montgomery step."""
+    m = C.c_int()
+    assert model.dec_choose(39, 10, 20, C.byref(m)) == 0
+    assert model.dec_choose(300, 1, 100, C.byref(m)) == 0
+    assert model.dec_choose(300, 2, 299, C.byref(m)) == 0
+    assert model.dec_choose(5000, 100, 5000, C.byref(m)) == 0
+    assert model.dec_choose(5000, 100, 4999, C.byref(m)) == 10 and m.value == DENSE
+    assert model.dec_choose(5000, 12, 4980, C.byref(m)) == 0
+    assert model.dec_choose(120000, 100, 60000, C.byref(m)) == 0
