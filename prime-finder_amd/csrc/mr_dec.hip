@@ -28,7 +28,7 @@ __device__ __forceinline__ void copy_form(Form &f, const Form *src)
 template <int LM>
 __global__ __launch_bounds__(G<LM>::THREADS) void exp_kernel(Args A, const double *__restrict__ tab, int steps)
 {
-    __shared__ double X[G<LM>::LDS];
+    __shared__ double X[lds_words<LM>()];
     __shared__ double bnd[3 * (G<LM>::THREADS / 64)];
     __shared__ Form f;
     const int c = slot_of(A);
@@ -46,10 +46,13 @@ __global__ __launch_bounds__(G<LM>::THREADS) void exp_kernel(Args A, const doubl
     const double *Nt = A.Nt + (size_t)c * A.tstride;
     double *park = A.park + (size_t)c * A.pstride;
     for (int i = threadIdx.x; i < Lw; i += G<LM>::THREADS) X[pd(i)] = dig[i];
+    if (threadIdx.x == 0) X[G<LM>::LDS] = 0.0;
     const int out = f.mode == TOP ? 0 : Lw;
     int off = 0;
     Terms u;
     load_terms(u, f);
+    const int q0 = threadIdx.x / G<LM>::TP;
+    const Fp F = prime_of(G<LM>::TP >= 64 ? uniform(q0) : q0);
     Twid<LM> h[hoisted<LM>() ? 2 : 1];
     if constexpr (hoisted<LM>()) {
         const int q = threadIdx.x / G<LM>::TP, t = threadIdx.x & (G<LM>::TP - 1);
@@ -57,9 +60,14 @@ __global__ __launch_bounds__(G<LM>::THREADS) void exp_kernel(Args A, const doubl
         h[1].load(tab + (2 * q + 1) * tab_size<LM>(), t);
     }
     __syncthreads();
+    // a limb of exponent bits at a time: loaded in every step, the barriers of
+    // the step waited for it
+    uint32_t bits = Nl[bp / 24] << (31 - bp % 24);
     for (int k = 0; k < steps && bp >= s; k++, bp--) {
-        const uint32_t bit = (Nl[bp / 24] >> (bp % 24)) & 1u;
-        square_step<LM>(X, bnd, f, u, tab, off, bit ? base : 1.0, h, Nt, park);
+        const uint32_t bit = bits >> 31;
+        bits <<= 1;
+        if (bp % 24 == 0 && bp) bits = Nl[bp / 24 - 1] << 8;
+        square_step<LM>(X, bnd, F, f, u, tab, off, bit ? base : 1.0, h, Nt, park);
         off = out;
     }
     for (int i = threadIdx.x; i < Lw; i += G<LM>::THREADS) dig[i] = X[pd(off + i)];
@@ -102,8 +110,10 @@ __device__ void canonical(double *X, int off, const Form &f)
         if (f.mode != TOP) X[pd(off)] -= 1.0;
         for (int k = 0; k < f.nt; k++) {
             const Term &t = f.t[k];
-            if (f.mode == TOP) X[pd(off + t.E + Lw)] -= t.c * t.ts;
-            else X[pd(off + t.E)] += t.c * t.ts;
+            const double c = f.mode == TOP ? -t.c : t.c, h = __builtin_trunc(c / t.tc);
+            const int E = off + t.E + (f.mode == TOP ? Lw : 0);
+            X[pd(E)] += (c - h * t.tc) * t.ts;
+            if (h != 0.0) X[pd(E + 1)] += h;
         }
         (void)carry_all(X, off, Lw);
     }
@@ -118,9 +128,12 @@ __device__ void canonical(double *X, int off, const Form &f)
             const int e = DIGITS * (t.E + Lw) + t.s - f.z, E = e / DIGITS, s = e % DIGITS;
             double ts = 1.0;
             for (int i = 0; i < s; i++) ts *= 10.0;
-            const double v = h * t.c, tc = B / ts, vh = __builtin_floor(v / tc);
-            X[pd(off + E)] += (v - vh * tc) * ts;
-            X[pd(off + E + 1)] += vh;
+            // h c < 10^18 at limb E, s digits up
+            const unsigned long long v = (unsigned long long)h * (unsigned long long)t.c;
+            const unsigned long long tc = (unsigned long long)(B / ts), lim = (unsigned long long)B;
+            X[pd(off + E)] += (double)(v % tc) * ts;
+            X[pd(off + E + 1)] += (double)(v / tc % lim);
+            if (v / tc >= lim) X[pd(off + E + 2)] += (double)(v / tc / lim);
         }
         (void)carry_all(X, off, Lw);
     }
@@ -129,7 +142,7 @@ __device__ void canonical(double *X, int off, const Form &f)
 template <int LM>
 __global__ __launch_bounds__(G<LM>::THREADS) void norm_kernel(Args A)
 {
-    __shared__ double X[G<LM>::XP];
+    __shared__ double X[G<LM>::XP + 2];
     __shared__ Form f;
     const int c = slot_of(A);
     if (A.path[c] != LM || A.pre[c]) return;
@@ -138,11 +151,12 @@ __global__ __launch_bounds__(G<LM>::THREADS) void norm_kernel(Args A)
     const int Lw = f.Lw, t = threadIdx.x;
     const double *dig = A.dig + (size_t)c * A.dstride;
     for (int i = t; i < G<LM>::M; i += G<LM>::THREADS) X[pd(i)] = i < Lw ? dig[i] : 0.0;
+    if (t == 0) X[G<LM>::XP] = 0.0;
     __syncthreads();
     const int off = f.mode == TOP ? 0 : Lw;
     Terms u;
     load_terms(u, f);
-    if (f.mode != TOP) fold<LM>(X, f, u, t);        // out of Montgomery form
+    if (f.mode != TOP) fold<LM>(X, G<LM>::XP, f, u, t);        // out of Montgomery form
     __syncthreads();
     if (t == 0) canonical(X, off, f);
     __syncthreads();
@@ -155,17 +169,18 @@ __global__ __launch_bounds__(G<LM>::THREADS) void norm_kernel(Args A)
 template <int LM>
 __global__ __launch_bounds__(G<LM>::THREADS) void prepare_kernel(Args A, const double *__restrict__ tab)
 {
-    __shared__ double X[G<LM>::LDS];
+    __shared__ double X[G<LM>::LDS + 2];
     __shared__ Form f;
     const int c = slot_of(A), t = threadIdx.x;
     if (A.form[c].lm != LM || A.form[c].mode != DENSE) return;
     copy_form<LM>(f, A.form + c);
     for (int i = t; i < G<LM>::M; i += G<LM>::THREADS) X[pd(i)] = i == 0 ? 1.0 : 0.0;
+    if (t == 0) X[G<LM>::LDS] = 0.0;
     __syncthreads();
     double *rec = A.park + (size_t)c * A.pstride;
     Terms u;
     load_terms(u, f);
-    fold<LM>(X, f, u, t, rec);
+    fold<LM>(X, G<LM>::LDS, f, u, t, rec);
     __syncthreads();
     for (int i = t; i < f.Lw; i += G<LM>::THREADS) X[pd(i)] = rec[i];
     __syncthreads();

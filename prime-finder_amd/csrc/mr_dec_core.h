@@ -35,7 +35,7 @@
 #define PF_DEC_HD inline
 namespace mr { namespace dec {
 int  tid();
-void sync_block();
+void sync_waves();
 void sync_wave();
 void sync_global();
 double lane_up(double x);          // the value of the lane below (lane 0: unspecified)
@@ -58,7 +58,7 @@ __device__ __forceinline__ int tid()
     return t;
 }
 // LDS hand-off between the waves of a block; global loads stay in flight.
-__device__ __forceinline__ void sync_block()
+__device__ __forceinline__ void sync_waves()
 {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
@@ -275,7 +275,7 @@ PF_DEC_FN void dft(double *x, const Fp &F)
 // only the first pass and its mirror need block barriers.
 constexpr int MIN_LM = 7, MAX_LM = 14;
 #ifndef PF_LR
-#define PF_LR(lm) (lm >= 14 ? 5 : lm >= 11 ? 4 : lm >= 9 ? 3 : 2)
+#define PF_LR(lm) (lm >= 14 ? 5 : lm >= 13 ? 4 : lm >= 11 ? 3 : 2)
 #endif
 constexpr int lr_of(int lm) { return PF_LR(lm); }
 
@@ -358,9 +358,12 @@ inline void build_tables(int lm, double *out)
 // Each term adds coef * (t shifted by 13 E + s digits); a fold round of TOP or
 // BOTTOM clears at most `gap` limbs, so that its targets lie outside its
 // sources.
+//
+// The multiple is a unit (Q's 1, or 10^D) and groups of up to six digits, so
+// that a candidate with k, j below 10^6 has one group for each.
 constexpr int MAX_TERMS = 16, TOP = 0, BOTTOM = 1, DENSE = 2;
 struct Term {
-    double c;                       // signed coefficient, |c| <= 99
+    double c;                       // signed coefficient, |c| < 10^6
     double ts, tc, itc;             // 10^s, 10^(13 - s) and its inverse
     int32_t E, s;                   // target offset in limbs (TOP: less Lw), digit shift
 };
@@ -368,8 +371,8 @@ struct Form {
     int32_t lm;                     // class, 0: not handled here
     int32_t mode, Lw, gap, nt;      // gap: limbs per fold round
     int32_t D, z, f;                // f = 13 Lw - D
-    int32_t pad;
-    Term t[MAX_TERMS];              // by offset
+    int32_t omin, omax;             // least and largest offset over the terms
+    Term t[MAX_TERMS];              // the unit (TOP: Q's 1, else 10^D), then the groups
 };
 
 // How a candidate with D digits whose Q has its terms (but the 1) at exponents
@@ -380,7 +383,7 @@ struct Form {
 // (dense_from rounds, measured), DENSE; its N' comes from BOTTOM's rounds, run
 // once.
 constexpr int MAX_ROUNDS = 64, MIN_DIGITS = 40, MAX_BASE = 511;
-constexpr int dense_from(int lm) { return lm <= 10 ? 4 : lm <= 12 ? 5 : 8; }
+constexpr int dense_from(int lm) { return lm <= 8 ? 7 : lm <= 11 ? 8 : 10; }
 struct Choice { int32_t lm, mode; };
 PF_DEC_HD Choice choose(int64_t D, int64_t lo, int64_t hi)
 {
@@ -407,29 +410,16 @@ PF_DEC_HD Choice choose(int64_t D, int64_t lo, int64_t hi)
 // order, unused ones zero): +1 at D, the rest negative.
 PF_DEC_HD void make_form(const int64_t *terms, int nterm, int64_t D, int lm, int mode, Form &f)
 {
-    int64_t e[3 * MAX_TERMS];
-    int g[3 * MAX_TERMS], n = 0;
-    for (int i = 0; i < nterm; i++) {           // Q in groups of two digits, by exponent
-        int64_t c = -terms[2 * i];
-        for (int64_t x = terms[2 * i + 1]; c > 0 && n < 3 * MAX_TERMS; x += 2, c /= 100) {
-            int at = n;
-            if (c % 100 == 0) continue;
-            for (; at > 0 && e[at - 1] > x; at--) { e[at] = e[at - 1]; g[at] = g[at - 1]; }
-            e[at] = x;
-            g[at] = (int)(c % 100);
-            n++;
-        }
-    }
-    int m = 0;
-    for (int i = 0; i < n; i++) {               // two neighbouring digits make a group
-        if (i + 1 < n && e[i + 1] == e[i] + 1 && g[i] <= 9 && g[i + 1] <= 9) {
-            e[m] = e[i];
-            g[m++] = g[i] + 10 * g[i + 1];
-            i++;
-        } else {
-            e[m] = e[i];
-            g[m++] = g[i];
-        }
+    int64_t e[MAX_TERMS * 2], g[MAX_TERMS * 2];
+    int n = 0;
+    for (int i = 0; i < nterm; i++) {           // Q less its 1, by exponent
+        int64_t c = -terms[2 * i], x = terms[2 * i + 1];
+        if (x == 0 && c > 0) c--;
+        if (c <= 0 || n == MAX_TERMS * 2) continue;
+        int at = n++;
+        for (; at > 0 && e[at - 1] > x; at--) { e[at] = e[at - 1]; g[at] = g[at - 1]; }
+        e[at] = x;
+        g[at] = c;
     }
     f.mode = mode;
     f.D = (int32_t)D;
@@ -437,8 +427,11 @@ PF_DEC_HD void make_form(const int64_t *terms, int nterm, int64_t D, int lm, int
     f.f = DIGITS * f.Lw - f.D;
     f.z = mode == TOP ? f.f : 0;
     f.nt = 0;
-    f.lm = m < MAX_TERMS ? lm : 0;
+    f.lm = lm;
+    f.omin = 1 << 30;
+    f.omax = -(1 << 30);
     auto put = [&](int64_t x, double c) {
+        if (f.nt == MAX_TERMS) { f.lm = 0; return; }
         Term &t = f.t[f.nt++];
         t.c = c;
         t.s = (int32_t)(x % DIGITS);
@@ -447,14 +440,38 @@ PF_DEC_HD void make_form(const int64_t *terms, int nterm, int64_t D, int lm, int
         for (int i = 0; i < t.s; i++) t.ts *= 10.0;
         t.tc = B / t.ts;                        // exact
         t.itc = t.ts / B;
+        f.omin = t.E < f.omin ? t.E : f.omin;
+        f.omax = t.E > f.omax ? t.E : f.omax;
     };
-    for (int i = 0; i < m && f.nt < MAX_TERMS; i++)     // offsets ascend
-        if (mode == TOP) put(e[i] + f.z, (double)g[i]);
-        else if (e[i] > 0) put(e[i], -(double)g[i]);
-    if (f.nt == 0) f.lm = 0;
-    f.gap = mode == TOP ? -f.t[f.nt ? f.nt - 1 : 0].E - 2 : f.t[0].E;
-    if (mode != TOP) put(D, 1.0);
+    put(mode == TOP ? f.z : D, 1.0);
+    for (int i = 0; i < n;) {                   // neighbouring digits below 10^6 together
+        int64_t c = 0, w = 1, at = e[i];
+        for (; i < n && e[i] - at <= 5; i++) {
+            for (w = 1; w < 1000000 && at + (w < 10 ? 0 : w < 100 ? 1 : w < 1000 ? 2 : w < 10000 ? 3 : w < 100000 ? 4 : 5) < e[i];) w *= 10;
+            if (c + g[i] * w >= 1000000) break;
+            c += g[i] * w;
+        }
+        if (c == 0) { c = g[i]; i++; }          // (10^6 itself, as k or j)
+        put(at + f.z, mode == TOP ? (double)c : -(double)c);
+    }
+    f.gap = mode == TOP ? -f.omax - 2 : f.omin;
     if (f.gap < 1) f.lm = 0;
+}
+
+// Where T waits during a DENSE squaring: in the LDS, behind the transforms (and
+// the zero word), where it fits; its limbs come back a barrier later instead of
+// a trip to memory.
+template <int LM>
+constexpr bool park_lds() { return LM <= 12; }
+template <int LM>
+constexpr int lds_words() { return G<LM>::LDS + 2 + (park_lds<LM>() ? G<LM>::M : 0); }
+
+// A block of one wave needs no barrier (its LDS operations stay in order).
+template <int LM>
+PF_DEC_FN void sync_block()
+{
+    if constexpr (G<LM>::THREADS > 64) sync_waves();
+    else sync_wave();
 }
 
 // ---- transform ----------------------------------------------------------------
@@ -657,27 +674,27 @@ PF_DEC_FN void run_finish(double (&z)[C], double i0, double i1, double ic, doubl
 }
 
 // ---- fold rounds ----------------------------------------------------------------
-// A target limb i gathers, per term with offset o, the shifted limb
-//   10^s (t[i-o] mod 10^(13-s)) + (t[i-o-1] div 10^(13-s))
-// (balanced remainders), so a limb's sum stays below 2^52.2: the terms sum to
-// at most 991 (20 digits in groups of two, and a 1) times 2^42.2.  Lanes take
-// consecutive targets, 62 new ones a wave: the quotient by 10^(13-s) comes
-// from the lane below, whose own limb it is (lane 0), and so does the carry
-// (lane 1).  The terms that fit (all five of a candidate with k, j below
-// 10^4) wait in scalar registers, and a target's limbs are all read before the
-// first is used: read one after the other, from terms in LDS, a round was a
-// chain of two LDS latencies per term.
-constexpr int NT = 5;               // terms held in registers
+// A target limb i gathers, per term with offset o, c times the shifted limb
+//   w = 10^s (t[i-o] mod 10^(13-s)) + (t[i-o-1] div 10^(13-s))
+// (balanced remainders).  c w < 2^63 splits exactly into a carry and a
+// remainder of at most B/2 (h = c w rounded, l = c w - h).  Lanes take
+// consecutive targets, 62 new ones a wave: the quotient by 10^(13-s) comes from
+// the lane below, whose own limb it is (lane 0), and so does the carry (lane
+// 1).  A round is one LDS latency and a chain of arithmetic: the unit and two
+// groups wait in scalar registers, a limb outside the sources is read from a
+// zero word (index zi) instead of branched around.  (Groups of two digits, terms
+// in LDS and branches took 1 800 cycles a round.)
+constexpr int NT = 2;               // groups held in registers
 struct Terms {
-    int nt, Lw, gap, mode, omin, omax, E[NT];
-    double c[NT], ts[NT], tc[NT], itc[NT];
+    int nt, Lw, gap, mode, omin, omax, E[NT + 1];
+    double c[NT + 1], ts[NT + 1], tc[NT + 1], itc[NT + 1];
 };
 PF_DEC_FN void load_terms(Terms &u, const Form &f)
 {
     u.nt = uniform(f.nt); u.Lw = uniform(f.Lw); u.gap = uniform(f.gap); u.mode = uniform(f.mode);
-    u.omin = uniform(f.t[0].E); u.omax = uniform(f.t[f.nt - 1].E);
+    u.omin = uniform(f.omin); u.omax = uniform(f.omax);
 #pragma unroll
-    for (int k = 0; k < NT; k++) {
+    for (int k = 0; k <= NT; k++) {
         const bool on = k < u.nt;
         const Term &m = f.t[on ? k : 0];
         u.E[k] = uniform(on ? m.E : 1 << 29);       // out of every range
@@ -686,42 +703,46 @@ PF_DEC_FN void load_terms(Terms &u, const Form &f)
     }
 }
 
-// Lane's target limb i of a strip starting at i0 (its lane 0): T[i] plus the
-// terms' multiples of the source limbs S[s0 .. s1), and its carry.
-PF_DEC_FN double gather(double acc, const double *S, int s0, int s1, int i0, int i, const Form &f,
-                        const Terms &u)
+// acc + the terms' multiples of the source limbs S[s0 .. s1) at target i; what
+// they carry out of the limb is added to car.  (Leaving out the terms that
+// reach no limb of a strip was slower: 100 000 digits, two rounds 54.6 -> 61 us.)
+PF_DEC_FN double gather(double acc, double &car, const double *S, int s0, int s1, int zi, int i,
+                        const Form &f, const Terms &u)
 {
-    double a[NT];
-    bool any[NT];
+    double a[NT + 1];
+    const unsigned n = (unsigned)(s1 - s0);
 #pragma unroll
-    for (int k = 0; k < NT; k++) {
+    for (int k = 0; k <= NT; k++) {
         const int p = i - u.E[k];
-        any[k] = i0 + 63 - u.E[k] >= s0 && i0 - u.E[k] <= s1;       // some lane's limb is a source
-        a[k] = 0.0;
-        if (any[k]) a[k] = p >= s0 && p < s1 ? S[pd(p)] : 0.0;
+        a[k] = S[(unsigned)(p - s0) < n ? pd(p) : zi];
     }
+    {
+        const double q = rint_(a[0] * u.itc[0]);
+        acc += fma_(u.ts[0], fma_(-q, u.tc[0], a[0]), lane_up(q));
+    }
+    auto group = [&](double x, double c, double ts, double tc, double itc) {
+        const double q = rint_(x * itc), w = fma_(ts, fma_(-q, tc, x), lane_up(q));
+        const double h = c * w, g = rint_(h * IB);
+        acc += fma_(-g, B, h) + fma_(c, w, -h);
+        car += g;
+    };
 #pragma unroll
-    for (int k = 0; k < NT; k++)
-        if (any[k]) {
-            const double q = rint_(a[k] * u.itc[k]);
-            acc = fma_(u.c[k], fma_(u.ts[k], fma_(-q, u.tc[k], a[k]), lane_up(q)), acc);
-        }
-    for (int k = NT; k < u.nt; k++) {
+    for (int k = 1; k <= NT; k++) group(a[k], u.c[k], u.ts[k], u.tc[k], u.itc[k]);
+    for (int k = NT + 1; k < u.nt; k++) {
         const Term &m = f.t[k];
         const int p = i - m.E;
-        const double b = p >= s0 && p < s1 ? S[pd(p)] : 0.0, q = rint_(b * m.itc);
-        acc = fma_(m.c, fma_(m.ts, fma_(-q, m.tc, b), lane_up(q)), acc);
+        group(S[(unsigned)(p - s0) < n ? pd(p) : zi], m.c, m.ts, m.tc, m.itc);
     }
     return acc;
 }
 
 // T (limbs in LDS, padded) -> the product reduced, at limbs [0, Lw) (TOP) or
 // [Lw, 2 Lw) (BOTTOM).  A round's targets lie outside its sources and span at
-// most Lw + 2 limbs.  (Cutting the targets into one window per group of terms
-// saved work but cost more in bookkeeping: 380 digits, two rounds 3.4 -> 6.4 us
-// a squaring.)  rec (BOTTOM on T = 1): the limbs cleared, N'.
+// most Lw + 2 limbs.  T[zi] is zero.  (Cutting the targets into one window per
+// group saved work but cost more in bookkeeping: 380 digits, two rounds 3.4 ->
+// 6.4 us a squaring.)  rec (BOTTOM on T = 1): the limbs cleared, N'.
 template <int LM>
-PF_DEC_FN void fold(double *T, const Form &f, const Terms &u, int t, double *rec = nullptr)
+PF_DEC_FN void fold(double *T, int zi, const Form &f, const Terms &u, int t, double *rec = nullptr)
 {
     constexpr int W = G<LM>::THREADS / 64, STEP = 62 * W, NI = (G<LM>::M / 2 + 1 + STEP) / STEP;
     const int lane = t & 63, wave = uniform(t >> 6);
@@ -740,19 +761,20 @@ PF_DEC_FN void fold(double *T, const Form &f, const Terms &u, int t, double *rec
         for (int n = 0; n < NI; n++) {
             const int i0 = lo + n * STEP + wave * 62 - 2, i = i0 + lane;
             if (i0 + 2 <= hi) {
-                const double acc = gather(i >= lo && i <= hi ? T[pd(i)] : 0.0,  // (limb lo - 1 keeps its carry)
-                                          T, s0, s1, i0, i, f, u);
+                double car = 0.0;
+                const double acc = gather(T[i >= lo && i <= hi ? pd(i) : zi],   // (limb lo - 1 keeps its carry)
+                                          car, T, s0, s1, zi, i, f, u);
                 const double c = i < hi ? rint_(acc * IB) : 0.0;    // (limb hi only takes one in)
-                out[n] = fma_(-c, B, acc) + lane_up(c);
+                out[n] = fma_(-c, B, acc) + lane_up(c + car);
             }
         }
-        sync_block();
+        sync_block<LM>();
 #pragma unroll
         for (int n = 0; n < NI; n++) {
             const int i = lo + n * STEP + wave * 62 - 2 + lane;
             if (lane > 1 && i <= hi) T[pd(i)] = out[n];
         }
-        sync_block();
+        sync_block<LM>();
     }
 }
 
@@ -761,19 +783,21 @@ PF_DEC_FN void fold(double *T, const Form &f, const Terms &u, int t, double *rec
 // their digits are at most B/2 and a little, so the multiple of B^Lw that they
 // sum to is zero, and only limb Lw - 1's carry is needed from them.
 template <int LM>
-PF_DEC_FN void dense_tail(double *X, const double *park, const Form &f, const Terms &u, int t)
+PF_DEC_FN void dense_tail(double *X, int zi, const double *park, const Form &f, const Terms &u, int t)
 {
     constexpr int W = G<LM>::THREADS / 64;
     const int lane = t & 63, wave = uniform(t >> 6), Lw = u.Lw;
-    for (int st = wave; st * 62 <= Lw; st += W) {
-        const int i0 = Lw + st * 62 - 2, i = i0 + lane;
+    for (int st = wave; st * 62 < Lw; st += W) {
+        const int i = Lw + st * 62 - 2 + lane;
         double acc = i >= Lw - 1 && i <= 2 * Lw ? park[i] : 0.0;
-        acc = gather(i == Lw - 1 ? acc - X[pd(i)] : acc, X, 0, Lw, i0, i, f, u);      // (N's -1 ends at Lw - 1)
+        if (st == 0) acc -= X[i == Lw - 1 ? pd(i) : zi];        // N's -1 ends at Lw - 1
+        double car = 0.0;
+        acc = gather(acc, car, X, 0, Lw, zi, i, f, u);
         const double c = rint_(acc * IB);
-        acc = fma_(-c, B, acc) + lane_up(c);
+        acc = fma_(-c, B, acc) + lane_up(c + car);
         if (lane > 1 && i < 2 * Lw) X[pd(i)] = acc;
     }
-    sync_block();
+    sync_block<LM>();
 }
 
 // ---- products ------------------------------------------------------------------
@@ -795,11 +819,12 @@ PF_DEC_FN Fp prime_of(int q)
 // or mul x times the number whose transform is at Nt (per prime M words), as
 // limbs [0, live + 2) at X (live: limbs of the result that are needed).  bnd: 3
 // words per wave.  tab: the class's tables, [prime][forward, inverse]; h: this
-// thread's hoisted twiddles (hoisted classes); keep: 3 M/2 words of global memory
+// thread's hoisted twiddles (hoisted classes), F0 its prime's constants (chosen
+// once: the choice costs as much as a pass); keep: 3 M/2 words of global memory
 // (SEQ classes).  Begins after a barrier and ends with one.
 template <int LM>
-PF_DEC_FN void product(double *X, double *bnd, int n, int off, int live, const double *tab, double mul,
-                       const Twid<LM> *h, const double *Nt, double *keep)
+PF_DEC_FN void product(double *X, double *bnd, const Fp &F0, int n, int off, int live, const double *tab,
+                       double mul, const Twid<LM> *h, const double *Nt, double *keep)
 {
     using g = G<LM>;
     constexpr int R = g::R, Q = g::M / R, C = g::C, TS = tab_size<LM>();
@@ -821,7 +846,7 @@ PF_DEC_FN void product(double *X, double *bnd, int n, int off, int live, const d
     };
     if constexpr (!g::SEQ) {
         const int q = g::TP >= 64 ? uniform(t / g::TP) : t / g::TP, tp = t & (g::TP - 1);
-        const Fp F = prime_of(q);
+        const Fp &F = F0;
         const double *tf = tab + 2 * q * TS, *ti = tf + TS;
         double *Y = X + q * g::XP, *Yb = Y + pd(tp);
         const double *Xd = X + pd(off + tp);
@@ -831,19 +856,19 @@ PF_DEC_FN void product(double *X, double *bnd, int n, int off, int live, const d
             const int i = tp + k * Q;
             v[k] = i < n ? Xd[po(k * Q)] : 0.0;
         }
-        sync_block();
+        sync_block<LM>();
         dft<g::LR, false, 10, 10, true>(v, F);      // |digit| < 2^42.4: 0.01 p
 #pragma unroll
         for (int k = 0; k < R; k++) Yb[po(k * Q)] = v[k];
-        sync_block();
+        sync_block<LM>();
         middle<LM, hoisted<LM>()>(Y, F, tf, ti, tp, h, Nt ? Nt + q * g::M : nullptr);
-        sync_block();
+        sync_block<LM>();
 #pragma unroll
         for (int k = 0; k < R; k++) v[k] = Yb[po(k * Q)];
         dft<g::LR, true, S1, S1>(v, F);
 #pragma unroll
         for (int k = 0; k < R; k++) Yb[po(k * Q)] = v[k];
-        sync_block();
+        sync_block<LM>();
         double z[C], o0 = 0.0, o1 = 0.0, *Xr = X + pd(t * C);
         const bool in = uniform(t & ~63) * C <= live + 2;       // waves above what is needed stay out
         oc = 0.0;
@@ -851,7 +876,7 @@ PF_DEC_FN void product(double *X, double *bnd, int n, int off, int live, const d
             run_digits<C, LM>(z, [&](int i) { return Xr[po(i)]; },
                               [&](int i) { return Xr[g::XP + po(i)]; }, mul, o0, o1, oc);
         hand_on(o0, o1, oc);
-        sync_block();
+        sync_block<LM>();
         take(t == 0);
         if (in) {
             run_finish<C>(z, i0, i1, ic, oc);
@@ -876,13 +901,13 @@ PF_DEC_FN void product(double *X, double *bnd, int n, int off, int live, const d
             if (q)
 #pragma unroll
                 for (int k = 0; k < R / 2; k++) v[k] = keep[g::M + k * g::TP + t];
-            sync_block();
+            sync_block<LM>();
             dft<g::LR, false, 10, 10, true>(v, F);
 #pragma unroll
             for (int k = 0; k < R; k++) Xb[po(k * Q)] = v[k];
-            sync_block();
+            sync_block<LM>();
             middle<LM, false>(X, F, tf, ti, t, nullptr, Nt ? Nt + q * g::M : nullptr);
-            sync_block();
+            sync_block<LM>();
 #pragma unroll
             for (int k = 0; k < R; k++) v[k] = Xb[po(k * Q)];
             dft<g::LR, true, S1, S1>(v, F);
@@ -908,7 +933,7 @@ PF_DEC_FN void product(double *X, double *bnd, int n, int off, int live, const d
                 run_digits<C, LM>(z, [&](int i) { return r0[i]; },
                                   [&](int i) { return Xr[po(h2 * H) + po(i)]; }, mul, o0, o1, oc);
             hand_on(o0, o1, oc);
-            sync_block();
+            sync_block<LM>();
             take(t == 0);
             if (t == 0) { i0 = b0; i1 = b1; ic = b2; }
             constexpr int E = 3 * (g::THREADS / 64) - 3;
@@ -918,34 +943,42 @@ PF_DEC_FN void product(double *X, double *bnd, int n, int off, int live, const d
 #pragma unroll
                 for (int i = 0; i < C; i++) Xr[po(h2 * H) + po(i)] = z[i];
             }
-            sync_block();
+            sync_block<LM>();
         }
     }
-    sync_block();
+    sync_block<LM>();
 }
 
-// mul x^2 (TOP) or mul x^2 R^-1 modulo N, x at limbs [off, off + Lw), left at
+// X: lds_words(), X[LDS] zero.  mul x^2 (TOP) or mul x^2 R^-1 modulo N, x at limbs [off, off + Lw), left at
 // limbs [0, Lw) or [Lw, 2 Lw).  DENSE: Nt the transform of N'.  park: global
 // memory, 2 Lw + 2 words (DENSE), then 3 M/2 (SEQ classes).
 template <int LM>
-PF_DEC_FN void square_step(double *X, double *bnd, const Form &f, const Terms &u, const double *tab, int off,
+PF_DEC_FN void square_step(double *X, double *bnd, const Fp &F, const Form &f, const Terms &u, const double *tab, int off,
                            double mul, const Twid<LM> *h, const double *Nt, double *park)
 {
     const int Lw = u.Lw;
     // one product instance: a second one would double the code and its registers
 #pragma clang loop unroll(disable)
     for (int second = 0;; second = 1) {
-        product<LM>(X, bnd, Lw, second ? 0 : off, second ? Lw : 2 * Lw, tab, second ? 1.0 : mul, h,
+        product<LM>(X, bnd, F, Lw, second ? 0 : off, second ? Lw : 2 * Lw, tab, second ? 1.0 : mul, h,
                     second ? Nt : nullptr, park + 2 * Lw + 2);
         if (second || u.mode != DENSE) break;
-        for (int i = tid(); i <= 2 * Lw; i += G<LM>::THREADS) park[i] = X[pd(i)];
-        sync_block();
+        if constexpr (park_lds<LM>()) {
+            for (int i = tid(); i <= 2 * Lw; i += G<LM>::THREADS) X[G<LM>::LDS + 2 + i] = X[pd(i)];
+        } else {
+            for (int i = tid(); i <= 2 * Lw; i += G<LM>::THREADS) park[i] = X[pd(i)];
+        }
+        sync_block<LM>();
     }
     if (u.mode == DENSE) {
-        sync_global();
-        dense_tail<LM>(X, park, f, u, tid());
+        if constexpr (park_lds<LM>()) {
+            dense_tail<LM>(X, G<LM>::LDS, X + G<LM>::LDS + 2, f, u, tid());
+        } else {
+            sync_global();
+            dense_tail<LM>(X, G<LM>::LDS, park, f, u, tid());
+        }
     } else {
-        fold<LM>(X, f, u, tid());
+        fold<LM>(X, G<LM>::LDS, f, u, tid());
     }
 }
 
@@ -968,11 +1001,11 @@ PF_DEC_FN void transform(double *X, int n, const double *tab, double *out)
         double *Y = g::SEQ ? X : X + q * g::XP, *Yb = Y + pd(tp);
 #pragma unroll
         for (int k = 0; k < R / 2; k++) v[k] = x[k];
-        sync_block();
+        sync_block<LM>();
         dft<g::LR, false, 10, 10, true>(v, F);
 #pragma unroll
         for (int k = 0; k < R; k++) Yb[po(k * Q)] = v[k];
-        sync_block();
+        sync_block<LM>();
         middle<LM, false>(Y, F, tab + 2 * q * TS, nullptr, tp, nullptr, nullptr, out + q * g::M);
     }
 }

@@ -876,21 +876,20 @@ __device__ void dec_start(double *dig, const dec::Form &f, uint32_t base)
     const u128 B = 10000000000000ull;
     double ten = 1.0, rho = 0.0;
     for (int i = 0; i < f.f; i++) ten *= 10.0;                  // exact: f <= 20
-    for (int k = 0; k < f.nt - 1; k++) {
+    for (int k = 1; k < f.nt; k++) {
         double v = -f.t[k].c;
         for (int e = dec::DIGITS * f.t[k].E + f.t[k].s; e < f.D && v > 1e-40; e++) v /= 10.0;
         rho += v;                                               // Q / 10^D < 0.1
     }
     const u128 q = (u128)(ten * rho / (1.0 - rho)), tenf = (u128)ten;
-    for (int k = -1; k < f.nt; k++) {       // Q's 1, its terms, then -q 10^D
-        const bool last = k == f.nt - 1;
-        const int e = k < 0 ? 0 : dec::DIGITS * f.t[k].E + f.t[k].s;
-        u128 w = last ? q * base : (tenf + q) * base * (uint32_t)(k < 0 ? 1.0 : -f.t[k].c);
-        for (int i = 0; i < e % dec::DIGITS; i++) w *= 10u;
-        for (int E = e / dec::DIGITS; w; E++, w /= B) {
-            const double v = (double)(uint64_t)(w % B);
-            dig[E] += last ? -v : v;
-        }
+    for (int k = -1; k < f.nt; k++) {       // Q's 1, -q 10^D, Q's groups
+        const int E = k < 0 ? 0 : f.t[k].E;
+        // below 10^21 10^6 2^9 < 2^100, s digits up: the lower limb's share and the rest
+        const u128 w = k == 0 ? q * base : (tenf + q) * base * (uint32_t)(k < 0 ? 1.0 : -f.t[k].c);
+        const u128 tc = (u128)(dec::B / (k < 0 ? 1.0 : f.t[k].ts));
+        dig[E] += (k == 0 ? -1.0 : 1.0) * (double)(uint64_t)(w % tc) * (k < 0 ? 1.0 : f.t[k].ts);
+        u128 r = w / tc;
+        for (int i = E + 1; r; i++, r /= B) dig[i] += (k == 0 ? -1.0 : 1.0) * (double)(uint64_t)(r % B);
     }
     double c = 0.0;
     const int ED = f.D / dec::DIGITS;
@@ -1212,7 +1211,7 @@ __global__ __launch_bounds__(THREADS) void dec_load_kernel(Dev D, Twiddles T, Co
         __syncthreads();
         if (threadIdx.x == 0) {
             dg[0] = 1ull;
-            for (int k = 0; k < f.nt - 1; k++) {
+            for (int k = 1; k < f.nt; k++) {
                 const uint64_t w = (uint64_t)f.t[k].ts, b = 10000000000000ull / w;
                 const uint64_t v = (uint64_t)-f.t[k].c;
                 dg[f.t[k].E] += v % b * w;

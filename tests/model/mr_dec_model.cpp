@@ -13,8 +13,8 @@ static std::barrier<> *g_block;
 static std::vector<std::unique_ptr<std::barrier<>>> *g_wave;
 static double g_lane[1024];
 int tid() { return t_id; }
-void sync_block() { g_block->arrive_and_wait(); }
-void sync_global() { sync_block(); }
+void sync_waves() { g_block->arrive_and_wait(); }
+void sync_global() { sync_waves(); }
 void sync_wave() { (*g_wave)[t_id >> 6]->arrive_and_wait(); }
 double lane_up(double x)
 {
@@ -30,9 +30,10 @@ template <int LM>
 static void run(const Form &f, double *dig, const double *mul, int steps)
 {
     using g = G<LM>;
-    std::vector<double> X(g::LDS, 1e300), bnd(3 * (g::THREADS / 64) + 3), tab(4 * tab_size<LM>()), Y(g::LDS), Nt(2 * g::M), park(3 * g::M + 4);
+    std::vector<double> X(lds_words<LM>(), 1e300), bnd(3 * (g::THREADS / 64) + 3), tab(4 * tab_size<LM>()), Y(g::LDS + 2), Nt(2 * g::M), park(3 * g::M + 4);
     build_tables(LM, tab.data());
     for (int i = 0; i < f.Lw; i++) X[pd(i)] = dig[i];
+    X[g::LDS] = Y[g::LDS] = 0.0;
     std::barrier<> blk(g::THREADS);
     std::vector<std::unique_ptr<std::barrier<>>> wv;
     for (int w = 0; w < g::THREADS / 64; w++) wv.emplace_back(new std::barrier<>(64));
@@ -53,16 +54,16 @@ static void run(const Form &f, double *dig, const double *mul, int steps)
             }
             if (f.mode == DENSE) {                  // N' and its transform
                 for (int i = t; i < g::M; i += g::THREADS) Y[pd(i)] = i ? 0.0 : 1.0;
-                sync_block();
-                fold<LM>(Y.data(), f, u, t, park.data());
-                sync_block();
+                sync_waves();
+                fold<LM>(Y.data(), g::LDS, f, u, t, park.data());
+                sync_waves();
                 for (int i = t; i < f.Lw; i += g::THREADS) Y[pd(i)] = park[i];
-                sync_block();
+                sync_waves();
                 transform<LM>(Y.data(), f.Lw, tab.data(), Nt.data());
-                sync_block();
+                sync_waves();
             }
             for (int s = 0; s < steps; s++) {
-                square_step<LM>(X.data(), bnd.data(), f, u, tab.data(), off, mul[s], h, Nt.data(), park.data());
+                square_step<LM>(X.data(), bnd.data(), prime_of(t / g::TP), f, u, tab.data(), off, mul[s], h, Nt.data(), park.data());
                 off = f.mode == TOP ? 0 : f.Lw;
             }
         });
