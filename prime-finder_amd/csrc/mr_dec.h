@@ -24,6 +24,35 @@ struct Args {
     int tstride, pstride;
 };
 
+// A context's Montgomery steps in base 2^43 (Gen): any odd moduli of L limbs.
+struct GenArgs {
+    Gen g;
+    const int32_t *path;        // [n] slots with a class here are not this path's (nullptr: none)
+    const uint32_t *N, *one;    // [n][nstride]
+    uint32_t *res;              // [n][nstride] 24-bit Montgomery residue (in)
+    int nstride;
+    const uint32_t *scr;        // [n][sstride] 24-bit limbs of N' mod 2^(24 L) and, half way
+    int sstride;                //   up, of R mod N (launch_gen_prepare reads them)
+    double *tab;                // [n][5][2 M] transforms of N, N', 2^(24 L) mod N, R mod N,
+                                //   an operand
+    double *dig;                // [n][dstride] result digits
+    int dstride;
+    double *park;               // [n][pstride]
+    int pstride;
+    int32_t *flag;              // [n] set: dig holds a new result
+    int32_t *bitpos;
+    const int32_t *sval;
+    const uint8_t *alive, *pre;
+    const uint32_t *base;
+};
+void launch_gen_prepare(const GenArgs &A, const double *tab, int n, hipStream_t st);
+// Up to `steps` exponent bits of every slot with a base of at most MAX_BASE; the
+// residue's digits (24-bit Montgomery form) to dig.
+void launch_gen_exp(const GenArgs &A, const double *tab, int n, int steps, hipStream_t st);
+// dig = a b 2^(-24 L) mod N (b == nullptr: a^2) for 24-bit limbs, one per uint64_t.
+void launch_gen_mul(const GenArgs &A, const double *tab, int n, const uint64_t *a, const uint64_t *b, int ld,
+                    hipStream_t st);
+
 // The class's twiddle tables on the current device (built once per device,
 // kept): [prime][forward, inverse].  nullptr on an error.
 const double *tables(int device, int lm);

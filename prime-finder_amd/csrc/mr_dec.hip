@@ -187,6 +187,138 @@ __global__ __launch_bounds__(G<LM>::THREADS) void prepare_kernel(Args A, const d
     transform<LM>(X, f.Lw, tab, A.Nt + (size_t)c * A.tstride);
 }
 
+// Digits of 2^sh times a number of 24-bit limbs into X's limbs [0, Lw).
+template <int LM, class W>
+__device__ __forceinline__ void gen_load(double *X, const W *v, int L, int sh, int Lw)
+{
+    for (int i = threadIdx.x; i < Lw; i += G<LM>::THREADS) X[pd(i)] = gen_limb(v, L, sh, i);
+    __syncthreads();
+}
+
+template <int LM>
+struct GenSlot {
+    double *Nt, *Np, *One, *OneR, *Y, *park;
+    __device__ GenSlot(const GenArgs &A, int c)
+    {
+        constexpr int P = 2 * G<LM>::M;
+        Nt = A.tab + (size_t)c * 5 * P;
+        Np = Nt + P;
+        One = Np + P;
+        OneR = One + P;
+        Y = OneR + P;
+        park = A.park + (size_t)c * A.pstride;
+    }
+};
+
+template <int LM>
+__device__ __forceinline__ void load_twid(Twid<LM> (&h)[hoisted<LM>() ? 2 : 1], const double *tab)
+{
+    if constexpr (hoisted<LM>()) {
+        const int q = threadIdx.x / G<LM>::TP, t = threadIdx.x & (G<LM>::TP - 1);
+        h[0].load(tab + 2 * q * tab_size<LM>(), t);
+        h[1].load(tab + (2 * q + 1) * tab_size<LM>(), t);
+    }
+}
+
+// The transforms a modulus needs: N, 2^(24 L) and R mod N, and N' = -N^-1 mod
+// R = 2^(43 Lw), by one Newton step y (2 + N y) from the N' mod 2^(24 L) at scr.
+template <int LM>
+__global__ __launch_bounds__(G<LM>::THREADS) void gen_prepare_kernel(GenArgs A, const double *__restrict__ tab)
+{
+    __shared__ double X[lds_words<LM>()];
+    __shared__ double bnd[3 * (G<LM>::THREADS / 64)];
+    const int c = blockIdx.x, L = A.g.L, Lw = A.g.Lw;
+    if (A.pre[c]) return;
+    GenSlot<LM> S(A, c);
+    const int q0 = threadIdx.x / G<LM>::TP;
+    const Fp F = prime_of(G<LM>::TP >= 64 ? uniform(q0) : q0);
+    Twid<LM> h[hoisted<LM>() ? 2 : 1];
+    load_twid<LM>(h, tab);
+    if (threadIdx.x == 0) X[G<LM>::LDS] = 0.0;
+    double *keep = S.park + 2 * Lw + 2;
+    gen_load<LM>(X, A.N + (size_t)c * A.nstride, L, 0, Lw);
+    transform<LM>(X, Lw, tab, S.Nt);
+    __syncthreads();
+    gen_load<LM>(X, A.one + (size_t)c * A.nstride, L, 0, Lw);
+    transform<LM>(X, Lw, tab, S.One);
+    __syncthreads();
+    const uint32_t *y = A.scr + (size_t)c * A.sstride;
+    gen_load<LM>(X, y + A.sstride / 2, L, 0, Lw);
+    transform<LM>(X, Lw, tab, S.OneR);
+    __syncthreads();
+    gen_load<LM>(X, y, L, 0, Lw);
+    product<Base2, LM>(X, bnd, F, Lw, 0, Lw, tab, 1.0, h, S.Nt, keep);
+    if (threadIdx.x == 0) X[0] += 2.0;
+    __syncthreads();
+    transform<LM>(X, Lw, tab, S.Y);
+    __syncthreads();
+    gen_load<LM>(X, y, L, 0, Lw);
+    product<Base2, LM>(X, bnd, F, Lw, 0, Lw, tab, 1.0, h, S.Y, keep);
+    transform<LM>(X, Lw, tab, S.Np);
+}
+
+template <int LM>
+__global__ __launch_bounds__(G<LM>::THREADS) void gen_exp_kernel(GenArgs A, const double *__restrict__ tab, int steps)
+{
+    __shared__ double X[lds_words<LM>()];
+    __shared__ double bnd[3 * (G<LM>::THREADS / 64)];
+    const int c = blockIdx.x, L = A.g.L, Lw = A.g.Lw;
+    if (!A.alive[c] || A.pre[c] || A.base[c] > (uint32_t)MAX_BASE || (A.path && A.path[c])) return;
+    const int s = A.sval[c];
+    int bp = A.bitpos[c];
+    if (bp < s) return;
+    const double base = (double)A.base[c];
+    const uint32_t *Nl = A.N + (size_t)c * A.nstride;
+    GenSlot<LM> S(A, c);
+    const int q0 = threadIdx.x / G<LM>::TP;
+    const Fp F = prime_of(G<LM>::TP >= 64 ? uniform(q0) : q0);
+    Twid<LM> h[hoisted<LM>() ? 2 : 1];
+    load_twid<LM>(h, tab);
+    // x 2^(24 L) 2^sh = x R, times R mod N: x R below N
+    gen_load<LM>(X, A.res + (size_t)c * A.nstride, L, A.g.sh, Lw);
+    mont_step<LM>(X, bnd, F, Lw, tab, 0, 1.0, h, S.OneR, S.Np, S.Nt, S.park);
+    uint32_t bits = Nl[bp / 24] << (31 - bp % 24);
+    bool last = false;
+    for (int k = 0; !last; k++) {
+        last = k == steps || bp < s;            // then times 2^(24 L) mod N: x R -> x 2^(24 L)
+        const uint32_t bit = bits >> 31;
+        mont_step<LM>(X, bnd, F, Lw, tab, Lw, bit && !last ? base : 1.0, h, last ? S.One : nullptr, S.Np, S.Nt,
+                      S.park);
+        bits <<= 1;
+        if (bp % 24 == 0 && bp) bits = Nl[bp / 24 - 1] << 8;
+        if (!last) bp--;
+    }
+    double *dig = A.dig + (size_t)c * A.dstride;
+    for (int i = threadIdx.x; i < Lw; i += G<LM>::THREADS) dig[i] = X[pd(Lw + i)];
+    if (threadIdx.x == 0) { A.bitpos[c] = bp; A.flag[c] = 1; }
+}
+
+template <int LM>
+__global__ __launch_bounds__(G<LM>::THREADS) void gen_mul_kernel(GenArgs A, const double *__restrict__ tab,
+                                                                 const uint64_t *a, const uint64_t *b, int ld)
+{
+    __shared__ double X[lds_words<LM>()];
+    __shared__ double bnd[3 * (G<LM>::THREADS / 64)];
+    const int c = blockIdx.x, L = A.g.L, Lw = A.g.Lw;
+    if (A.pre[c]) return;
+    GenSlot<LM> S(A, c);
+    const int q0 = threadIdx.x / G<LM>::TP;
+    const Fp F = prime_of(G<LM>::TP >= 64 ? uniform(q0) : q0);
+    Twid<LM> h[hoisted<LM>() ? 2 : 1];
+    load_twid<LM>(h, tab);
+    if (b) {
+        gen_load<LM>(X, b + (size_t)c * ld, L, 0, Lw);
+        transform<LM>(X, Lw, tab, S.Y);
+        __syncthreads();
+    }
+    // 2^sh a b R^-1 = a b 2^(-24 L)
+    gen_load<LM>(X, a + (size_t)c * ld, L, b ? A.g.sh : A.g.sh / 2, Lw);
+    mont_step<LM>(X, bnd, F, Lw, tab, 0, !b && (A.g.sh & 1) ? 2.0 : 1.0, h, b ? S.Y : nullptr, S.Np, S.Nt, S.park);
+    double *dig = A.dig + (size_t)c * A.dstride;
+    for (int i = threadIdx.x; i < Lw; i += G<LM>::THREADS) dig[i] = X[pd(Lw + i)];
+    if (threadIdx.x == 0) A.flag[c] = 1;
+}
+
 __global__ void form_kernel(const int32_t *list, int n, const int64_t *terms, int nterm,
                             const int32_t *choice, Form *form, uint32_t *err)
 {
@@ -260,6 +392,31 @@ void launch_norm(int lm, const Args &A, int n, hipStream_t st)
     by_class(lm, [&](auto c) {
         constexpr int LM = decltype(c)::value;
         norm_kernel<LM><<<n, G<LM>::THREADS, 0, st>>>(A);
+    });
+}
+
+void launch_gen_prepare(const GenArgs &A, const double *tab, int n, hipStream_t st)
+{
+    by_class(A.g.lm, [&](auto c) {
+        constexpr int LM = decltype(c)::value;
+        gen_prepare_kernel<LM><<<n, G<LM>::THREADS, 0, st>>>(A, tab);
+    });
+}
+
+void launch_gen_exp(const GenArgs &A, const double *tab, int n, int steps, hipStream_t st)
+{
+    by_class(A.g.lm, [&](auto c) {
+        constexpr int LM = decltype(c)::value;
+        gen_exp_kernel<LM><<<n, G<LM>::THREADS, 0, st>>>(A, tab, steps);
+    });
+}
+
+void launch_gen_mul(const GenArgs &A, const double *tab, int n, const uint64_t *a, const uint64_t *b, int ld,
+                    hipStream_t st)
+{
+    by_class(A.g.lm, [&](auto c) {
+        constexpr int LM = decltype(c)::value;
+        gen_mul_kernel<LM><<<n, G<LM>::THREADS, 0, st>>>(A, tab, a, b, ld);
     });
 }
 

@@ -144,8 +144,15 @@ constexpr Fp FP0 = make_fp(Y0, P0), FP1 = make_fp(Y1, P1);
 // CRT of coefficients V, |V| < P0 P1 / 2: V = r0 + P0 u with
 // u = (r1 - r0) P0^-1 mod P1; then V in base B from P0 = CA B + CA0.
 constexpr double INV01 = balanced(powmod(P0 % P1, P1 - 2, P1), P1);
-constexpr double CA = (double)((P0 + 5000000000000ull) / 10000000000000ull);
-constexpr double CA0 = (double)((int64_t)P0 - (int64_t)CA * 10000000000000ll);
+struct Base10 {                     // search-form candidates
+    static constexpr double B = 1e13, IB = 1e-13, CA = (double)((P0 + 5000000000000ull) / 10000000000000ull),
+                            CA0 = (double)((int64_t)P0 - (int64_t)CA * 10000000000000ll);
+};
+struct Base2 {                      // any odd modulus
+    static constexpr int BITS = 43;
+    static constexpr double B = 8796093022208.0, IB = 1.0 / B,
+                            CA = (double)((P0 + (1ull << 42)) >> 43), CA0 = (double)((int64_t)P0 - ((int64_t)CA << 43));
+};
 
 // a w mod p for |w| <= p/2: |result| <= (0.5 + 0.125 |a|/p) p, exact while
 // |a w| / p < 2^52 (q's three roundings lose at most 0.125 |a|/p).
@@ -611,7 +618,7 @@ PF_DEC_FN void middle(double *X, const Fp &F, const double *tf, const double *ti
 struct Split { double d0, d1, d2; };
 // The coefficient V = M^-1 (r0 mod P0, r1 mod P1), |V| < 2^97.4, in base B.
 // M^-1 a = a1 - a0 (p - 1)/M for a = a1 M + a0.
-template <int LM>
+template <class S, int LM>
 PF_DEC_FN Split crt_split(double r0, double r1)
 {
     constexpr double Md = (double)(1 << LM), iM = 1.0 / Md;
@@ -623,17 +630,17 @@ PF_DEC_FN Split crt_split(double r0, double r1)
     constexpr double p1 = (double)P1, ip1 = 1.0 / (double)P1;
     double u = mulmod_d(x1 - x0, INV01, p1, ip1);
     if (LM > 13) u = reduce(u, p1, ip1);        // |V / P0| reaches 0.43 P1: q's rounding may be one off
-    const double u1 = rint_(u * IB), u0 = fma_(-u1, B, u);
-    const double h = u0 * CA0, l = fma_(u0, CA0, -h);
-    const double q = rint_(h * IB);
-    const double s0 = (fma_(-q, B, h) + l) + x0;
-    const double q0 = rint_(s0 * IB);
-    const double s1 = fma_(CA, u0, fma_(CA0, u1, q + q0));
-    const double q1 = rint_(s1 * IB);
+    const double u1 = rint_(u * S::IB), u0 = fma_(-u1, S::B, u);
+    const double h = u0 * S::CA0, l = fma_(u0, S::CA0, -h);
+    const double q = rint_(h * S::IB);
+    const double s0 = (fma_(-q, S::B, h) + l) + x0;
+    const double q0 = rint_(s0 * S::IB);
+    const double s1 = fma_(S::CA, u0, fma_(S::CA0, u1, q + q0));
+    const double q1 = rint_(s1 * S::IB);
     Split o;
-    o.d0 = fma_(-q0, B, s0);
-    o.d1 = fma_(-q1, B, s1);
-    o.d2 = fma_(CA, u1, q1);
+    o.d0 = fma_(-q0, S::B, s0);
+    o.d1 = fma_(-q1, S::B, s1);
+    o.d2 = fma_(S::CA, u1, q1);
     return o;
 }
 
@@ -641,13 +648,13 @@ PF_DEC_FN Split crt_split(double r0, double r1)
 // d2[i-2]) as far as the run knows them.  o0, o1: what the next run's first
 // two limbs still get; oc: the carry out of z[C-1] (run_finish takes the same
 // one out of it).
-template <int C, int LM, class LD0, class LD1>
+template <class S, int C, int LM, class LD0, class LD1>
 PF_DEC_FN void run_digits(double (&z)[C], LD0 r0, LD1 r1, double mul, double &o0, double &o1, double &oc)
 {
     double p1 = 0.0, p2 = 0.0, q2 = 0.0;        // d1[i-1], d2[i-1], d2[i-2]
 #pragma unroll
     for (int i = 0; i < C; i++) {
-        const Split s = crt_split<LM>(r0(i), r1(i));
+        const Split s = crt_split<S, LM>(r0(i), r1(i));
         z[i] = mul * (s.d0 + p1 + q2);
         p1 = s.d1;
         q2 = p2;
@@ -655,11 +662,11 @@ PF_DEC_FN void run_digits(double (&z)[C], LD0 r0, LD1 r1, double mul, double &o0
     }
     o0 = mul * (p1 + q2);
     o1 = mul * p2;
-    oc = rint_(z[C - 1] * IB);
+    oc = rint_(z[C - 1] * S::IB);
 }
 // Second half: with the run below's o0, o1, oc.  Limbs stay below
 // B/2 + 2^12: |z| <= 512 (B + 2^12), an exact carry of at most 2^10 each.
-template <int C>
+template <class S, int C>
 PF_DEC_FN void run_finish(double (&z)[C], double i0, double i1, double ic, double oc)
 {
     z[0] += i0;
@@ -667,8 +674,8 @@ PF_DEC_FN void run_finish(double (&z)[C], double i0, double i1, double ic, doubl
     double cin = ic;
 #pragma unroll
     for (int i = 0; i < C; i++) {
-        const double c = i == C - 1 ? oc : rint_(z[i] * IB);
-        z[i] = fma_(-c, B, z[i]) + cin;
+        const double c = i == C - 1 ? oc : rint_(z[i] * S::IB);
+        z[i] = fma_(-c, S::B, z[i]) + cin;
         cin = c;
     }
 }
@@ -822,7 +829,7 @@ PF_DEC_FN Fp prime_of(int q)
 // thread's hoisted twiddles (hoisted classes), F0 its prime's constants (chosen
 // once: the choice costs as much as a pass); keep: 3 M/2 words of global memory
 // (SEQ classes).  Begins after a barrier and ends with one.
-template <int LM>
+template <class S, int LM>
 PF_DEC_FN void product(double *X, double *bnd, const Fp &F0, int n, int off, int live, const double *tab,
                        double mul, const Twid<LM> *h, const double *Nt, double *keep)
 {
@@ -873,13 +880,13 @@ PF_DEC_FN void product(double *X, double *bnd, const Fp &F0, int n, int off, int
         const bool in = uniform(t & ~63) * C <= live + 2;       // waves above what is needed stay out
         oc = 0.0;
         if (in)
-            run_digits<C, LM>(z, [&](int i) { return Xr[po(i)]; },
+            run_digits<S, C, LM>(z, [&](int i) { return Xr[po(i)]; },
                               [&](int i) { return Xr[g::XP + po(i)]; }, mul, o0, o1, oc);
         hand_on(o0, o1, oc);
         sync_block<LM>();
         take(t == 0);
         if (in) {
-            run_finish<C>(z, i0, i1, ic, oc);
+            run_finish<S, C>(z, i0, i1, ic, oc);
 #pragma unroll
             for (int i = 0; i < C; i++) Xr[po(i)] = z[i];
         }
@@ -930,7 +937,7 @@ PF_DEC_FN void product(double *X, double *bnd, const Fp &F0, int n, int off, int
             const double *r0 = keep + h2 * H + t * C;
             oc = 0.0;
             if (in)
-                run_digits<C, LM>(z, [&](int i) { return r0[i]; },
+                run_digits<S, C, LM>(z, [&](int i) { return r0[i]; },
                                   [&](int i) { return Xr[po(h2 * H) + po(i)]; }, mul, o0, o1, oc);
             hand_on(o0, o1, oc);
             sync_block<LM>();
@@ -939,7 +946,7 @@ PF_DEC_FN void product(double *X, double *bnd, const Fp &F0, int n, int off, int
             constexpr int E = 3 * (g::THREADS / 64) - 3;
             b0 = bnd[E]; b1 = bnd[E + 1]; b2 = bnd[E + 2];
             if (in) {
-                run_finish<C>(z, i0, i1, ic, oc);
+                run_finish<S, C>(z, i0, i1, ic, oc);
 #pragma unroll
                 for (int i = 0; i < C; i++) Xr[po(h2 * H) + po(i)] = z[i];
             }
@@ -960,7 +967,7 @@ PF_DEC_FN void square_step(double *X, double *bnd, const Fp &F, const Form &f, c
     // one product instance: a second one would double the code and its registers
 #pragma clang loop unroll(disable)
     for (int second = 0;; second = 1) {
-        product<LM>(X, bnd, F, Lw, second ? 0 : off, second ? Lw : 2 * Lw, tab, second ? 1.0 : mul, h,
+        product<Base10, LM>(X, bnd, F, Lw, second ? 0 : off, second ? Lw : 2 * Lw, tab, second ? 1.0 : mul, h,
                     second ? Nt : nullptr, park + 2 * Lw + 2);
         if (second || u.mode != DENSE) break;
         if constexpr (park_lds<LM>()) {
@@ -980,6 +987,95 @@ PF_DEC_FN void square_step(double *X, double *bnd, const Fp &F, const Form &f, c
     } else {
         fold<LM>(X, G<LM>::LDS, f, u, tid());
     }
+}
+
+// ---- any odd modulus ------------------------------------------------------------
+// The same transforms in base 2^43 carry the Montgomery step of a modulus
+// without structure: T = mul x y, m = T N' mod R, (T + m N) / R with R =
+// 2^(43 Lw), three products, digits balanced as above.  R is at least 2^16
+// times the 2^(24 L) of the 24-bit form (sh = 43 Lw - 24 L), so that |x| stays
+// below N whatever the base (below 512) multiplied in.
+struct Gen {
+    int32_t lm, Lw, sh, L;
+};
+PF_DEC_HD Gen gen_of(int L)
+{
+    Gen g = {0, 0, 0, L};
+    g.Lw = (24 * L + 16 + Base2::BITS - 1) / Base2::BITS;
+    g.sh = Base2::BITS * g.Lw - 24 * L;
+    for (int lm = MIN_LM; lm <= MAX_LM && !g.lm; lm++)
+        if ((1 << lm) >= 2 * g.Lw + 4) g.lm = lm;
+    return g;
+}
+
+// Limb i (43 bits, balanced) of 2^sh times the number of n 24-bit limbs at v
+// (one per word W).
+template <class W>
+PF_DEC_FN double gen_limb(const W *v, int n, int sh, int i)
+{
+    auto raw = [&](int k) {
+        const int at = 43 * k - sh;                     // first bit, maybe below 0
+        if (at + 43 <= 0) return 0ull;
+        const int j = at >= 0 ? at / 24 : -1, o = at - 24 * j;      // o in [0, 24), or from limb -1
+        unsigned long long x = 0;
+        const unsigned long long a0 = j >= 0 && j < n ? v[j] & 0xFFFFFF : 0, a1 = j + 1 < n ? v[j + 1] & 0xFFFFFF : 0,
+                                 a2 = j + 2 < n ? v[j + 2] & 0xFFFFFF : 0;
+        if (at >= 0) {
+            x = (a0 >> o) | (a1 << (24 - o)) | (a2 << (48 - o));
+        } else {                                        // starts -at bits below the number
+            const int d = -at;                          // 1 .. 42
+            const unsigned long long b0 = n > 0 ? v[0] & 0xFFFFFF : 0, b1 = n > 1 ? v[1] & 0xFFFFFF : 0;
+            x = (b0 << d) | (d < 19 ? b1 << (24 + d) : 0ull);
+        }
+        return x & ((1ull << 43) - 1);
+    };
+    const unsigned long long x = raw(i), y = i > 0 ? raw(i - 1) : 0ull, h = 1ull << 42;
+    return (double)(long long)x - (x >= h ? Base2::B : 0.0) + (y >= h ? 1.0 : 0.0);
+}
+
+// x at X's limbs [off, off + Lw) -> mul x^2 R^-1, or mul x y R^-1 for the
+// transform y0 of y, at limbs [Lw, 2 Lw).  Np, Nt: transforms of N' and N.
+// park: global memory, 2 Lw + 2 words (from class 13), then 3 M/2 (SEQ).
+template <int LM>
+PF_DEC_FN void mont_step(double *X, double *bnd, const Fp &F, int Lw, const double *tab, int off, double mul,
+                         const Twid<LM> *h, const double *y0, const double *Np, const double *Nt, double *park)
+{
+    constexpr int W = G<LM>::THREADS / 64;
+    double *Tl = X + G<LM>::LDS + 2;
+#pragma clang loop unroll(disable)
+    for (int k = 0; k < 3; k++) {
+        product<Base2, LM>(X, bnd, F, Lw, k ? 0 : off, k == 1 ? Lw : 2 * Lw, tab, k ? 1.0 : mul, h,
+                           k == 0 ? y0 : k == 1 ? Np : Nt, park + 2 * Lw + 2);
+        if (k) continue;
+        for (int i = Lw - 1 + tid(); i < 2 * Lw; i += G<LM>::THREADS) {
+            if constexpr (park_lds<LM>()) Tl[i] = X[pd(i)];
+            else park[i] = X[pd(i)];
+        }
+        sync_block<LM>();
+    }
+    if constexpr (!park_lds<LM>()) sync_global();
+    // the limbs below Lw come to zero (as in dense_tail); lane 0 gives the carry
+    constexpr int NI = (G<LM>::M / 2 + 63 * W - 1) / (63 * W);
+    const int t = tid(), lane = t & 63, wave = uniform(t >> 6);
+    double out[NI];
+#pragma unroll
+    for (int n = 0; n < NI; n++) {
+        const int i = Lw - 1 + (wave + n * W) * 63 + lane;
+        double acc = 0.0;
+        if (i < 2 * Lw) {
+            if constexpr (park_lds<LM>()) acc = X[pd(i)] + Tl[i];
+            else acc = X[pd(i)] + park[i];
+        }
+        const double c = rint_(acc * Base2::IB);
+        out[n] = fma_(-c, Base2::B, acc) + lane_up(c);
+    }
+    sync_block<LM>();
+#pragma unroll
+    for (int n = 0; n < NI; n++) {
+        const int i = Lw - 1 + (wave + n * W) * 63 + lane;
+        if (lane > 0 && i < 2 * Lw) X[pd(i)] = out[n];
+    }
+    sync_block<LM>();
 }
 
 // The transform of the n digits at X's limbs [0, n), per prime M words at out.

@@ -71,6 +71,7 @@ struct Dev {                    // per-batch device state (kernel argument)
     int dstride;
     double *decNt, *park;       // [n][tstride], [n][pstride]: see dec::Args
     int tstride, pstride;
+    int gen;                    // 1: rounds with bases up to dec::MAX_BASE run in dec::Gen's step
 };
 
 __device__ __forceinline__ int slot_id(const Dev &D)
@@ -847,6 +848,7 @@ __global__ __launch_bounds__(THREADS) void setup_kernel(Dev D, Twiddles T, Const
         }
     }
     to_fft<LOGM>(sm, T, K, y, L, Npf, fsave);
+    store_vec<C>(y, scr, L, 0);                        // (dec::GenArgs)
 
     // R mod N: 2^nbits - N, then doubled (24 L - nbits) times mod N.
     {
@@ -981,6 +983,7 @@ __global__ __launch_bounds__(THREADS) void exp_kernel(Dev D, Twiddles T, Consts 
     int bp = D.bitpos[c];
     if (bp < s) return;
     const uint32_t base = D.base[c];
+    if (D.gen && base <= (uint32_t)dec::MAX_BASE) return;
     const int L = D.Ls[c];
     const uint32_t *Nl = D.N + (size_t)c * D.stride;
     uint32_t r[C];
@@ -1267,6 +1270,99 @@ __global__ __launch_bounds__(THREADS) void dec_load_kernel(Dev D, Twiddles T, Co
     }
 }
 
+// R mod N of dec::Gen's step, 2^sh times the 24-bit form's, at the upper half
+// of the slot's scratch.
+template <int LOGM>
+__global__ __launch_bounds__(THREADS) void gen_one_kernel(Dev D, int sh)
+{
+    constexpr int M = G<LOGM>::M, C = G<LOGM>::C;
+    __shared__ Scratch sc;
+    const int c = blockIdx.x, L = D.Ls[c];
+    if (D.pre[c]) return;
+    uint32_t r[C];
+    load_vec<C>(r, D.one + (size_t)c * D.stride, L, 0);
+    for (int k = 0; k < sh; k++) {
+        add_vec<C>(r, r, 0u, sc);
+        reduce_once<C>(r, D.N + (size_t)c * D.stride, L, 0, sc);
+    }
+    store_vec<C>(r, D.scr + (size_t)c * 2 * M + M, L, 0);
+}
+
+// A new result of dec::Gen's step (signed digits of base 2^43, above -N and
+// below 2 N) as a number below N: to D.res, or, with out, to one limb per
+// uint64_t.  Slots decided without rounds get zeros at out.  Vectors pass
+// through the LDS so that memory sees consecutive lanes on consecutive words (a
+// thread's run of limbs straight from and to memory: 38 us for 256 numbers of
+// 50 000 digits).
+template <int LOGM>
+__global__ __launch_bounds__(THREADS) void gen_store_kernel(Dev D, dec::Gen g, const double *dig, int dstride,
+                                                            int32_t *flag, uint64_t *out, int ld)
+{
+    constexpr int C = G<LOGM>::C;
+    __shared__ uint64_t buf[(Lds<LOGM>::MP + 1) / 2];       // MP limbs, or Lw < MP / 2 digits
+    __shared__ Scratch sc;
+    const int c = blockIdx.x, L = D.Ls[c], Lw = g.Lw, t = threadIdx.x;
+    uint32_t *lb = (uint32_t *)buf;
+    uint64_t *o64 = out + (size_t)c * ld;
+    if (out && D.pre[c]) {
+        for (int i = t; i < ld; i += THREADS) o64[i] = 0u;
+        return;
+    }
+    if (!flag[c]) return;
+    // digits + 2^43 (less the 1 the digit below took), all positive: the value +
+    // 2^(43 Lw)
+    dig += (size_t)c * dstride;
+    constexpr int64_t B = 1ll << 43;
+    for (int i = t; i < Lw; i += THREADS) buf[i] = (uint64_t)((int64_t)dig[i] + B - (i > 0 ? 1 : 0));
+    __syncthreads();
+    const int p0 = tid_() * C;
+    auto digit = [&](int i) { return i < Lw ? buf[i] : 0ull; };
+    uint32_t r[C], n[C];
+#pragma unroll
+    for (int i = 0; i < C; i++) {
+        const int at = 24 * (p0 + i), k = at / 43, o = at - 43 * k;     // bit o of digit k
+        uint32_t x = 0u;
+        if (k <= Lw) {
+            x = (uint32_t)(digit(k) >> o) & LIMB_MASK;
+            if (o > 19) x += (uint32_t)(digit(k + 1) << (43 - o)) & LIMB_MASK;
+            if (o == 0 && k > 0) x += (uint32_t)(digit(k - 1) >> 43);   // a digit's bit 43
+        }
+        r[i] = x;
+    }
+    mul_small_vec<C>(r, 1u, sc);                            // carries
+    const int top = 43 * Lw;                                // set: the value is not negative
+    bool pos = false;
+#pragma unroll
+    for (int i = 0; i < C; i++)
+        if (p0 + i == top / 24 && (r[i] >> (top % 24))) { pos = true; r[i] &= (1u << (top % 24)) - 1u; }
+    pos = block_any(pos, sc);
+    const uint32_t *Nl = D.N + (size_t)c * D.stride;
+    for (int i = t; i < L; i += THREADS) lb[px(i)] = Nl[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < C; i++) n[i] = p0 + i < L ? lb[px(p0 + i)] : 0u;
+    __syncthreads();
+    if (pos) {                                              // below 2 N
+        uint32_t d[C];
+        if (!sub_vec<C>(d, r, n, sc)) {
+#pragma unroll
+            for (int i = 0; i < C; i++) r[i] = d[i];
+        }
+    } else {                                                // value + 2^(43 Lw): + N passes 2^(43 Lw)
+        add_vec<C>(r, n, 0u, sc);
+    }
+#pragma unroll
+    for (int i = 0; i < C; i++)
+        if (p0 + i < L) lb[px(p0 + i)] = r[i];
+    __syncthreads();
+    uint32_t *res = D.res + (size_t)c * D.stride;
+    if (out)
+        for (int i = t; i < ld; i += THREADS) o64[i] = i < L ? lb[px(i)] : 0u;
+    else
+        for (int i = t; i < L; i += THREADS) res[i] = lb[px(i)];
+    if (t == 0) flag[c] = 0;
+}
+
 // op AR_MUL: out = A B R^-1 mod N; AR_SQ: A^2 R^-1; AR_CHECK: flag = (A ==
 // R mod N or A == (N-1) R mod N); AR_R2: r2 = R^2 mod N;
 // AR_TORES: out = A R mod N (A < N, times r2); AR_FROMRES: out = A R^-1 mod
@@ -1460,6 +1556,12 @@ struct mr_ctx {
     // whether some take the Montgomery step (bit 0)
     uint32_t classes = 1u;
     const double *tab[dec::MAX_LM + 1] = {};
+    // dec::Gen's step for the others (gen.lm 0: not set up)
+    dec::Gen gen = {0, 0, 0, 0};
+    const double *gen_tw = nullptr;
+    double *gen_tab = nullptr, *gen_dig = nullptr, *gen_park = nullptr;
+    int32_t *gen_flag = nullptr;
+    int gen_pstride = 0;
 };
 
 namespace {
@@ -1607,6 +1709,39 @@ int ctx_alloc_all(mr_ctx *x, long bits, int min_logm, bool with_dec = false, int
     return 0;
 }
 
+dec::GenArgs gen_args(const mr_ctx *x)
+{
+    const Dev &d = x->d;
+    return dec::GenArgs{x->gen, d.path, d.N, d.one, d.res, d.stride, d.scr, 2 << x->logm, x->gen_tab,
+                        x->gen_dig, x->gen.Lw + 2, x->gen_park, x->gen_pstride, x->gen_flag, d.bitpos,
+                        d.sval, d.alive, d.pre, d.base};
+}
+
+// Where it can, a context's Montgomery steps run in dec::Gen's form: arrays and
+// the moduli's transforms, after setup_kernel.
+int gen_setup(mr_ctx *x)
+{
+    dec::Gen g = dec::gen_of(x->L);
+    if (!g.lm || g_min_logm > MIN_LOGM) return 0;
+    const size_t n = (size_t)x->n, M = (size_t)1 << g.lm;
+    if (!(x->gen_tw = dec::tables(x->device, g.lm))) return -2;
+    x->gen_pstride = 2 * g.Lw + 2 + (g.lm > 13 ? 3 << g.lm >> 1 : 0);
+    if (ctx_alloc(x, (void **)&x->gen_tab, n * 10 * M * sizeof(double)) != 0 ||
+        ctx_alloc(x, (void **)&x->gen_dig, n * (g.Lw + 2) * sizeof(double)) != 0 ||
+        ctx_alloc(x, (void **)&x->gen_park, n * x->gen_pstride * sizeof(double)) != 0 ||
+        ctx_alloc(x, (void **)&x->gen_flag, n * sizeof(int32_t)) != 0)
+        return -2;
+    x->gen = g;
+    x->d.gen = 1;
+    (void)dispatch_logm(x->logm, [&](auto lg) {
+        gen_one_kernel<decltype(lg)::value><<<x->n, THREADS, 0, x->st>>>(x->d, g.sh);
+        return 0;
+    });
+    dec::launch_gen_prepare(gen_args(x), x->gen_tw, x->n, x->st);
+    MR_CHECK(hipGetLastError());
+    return 0;
+}
+
 // Per-candidate constants once the moduli are resident in d.N.
 int ctx_finish(mr_ctx *x)
 {
@@ -1618,6 +1753,8 @@ int ctx_finish(mr_ctx *x)
     });
     if (rc) return rc;
     MR_CHECK(hipGetLastError());
+    rc = gen_setup(x);
+    if (rc) return rc;
     uint32_t err = 0;
     MR_CHECK(hipMemcpyAsync(&err, x->d.err, 4, hipMemcpyDeviceToHost, x->st));
     x->sval.resize(n);
@@ -1724,25 +1861,34 @@ extern "C" int mr_ctx_moduli(const mr_ctx_t *x, uint32_t *out)
 namespace {
 
 // One chunk of squarings over the whole context: every class its candidates
-// run in, and the Montgomery step where some need it (all bases above
-// MAX_BASE do).
+// run in (bit lm), and for the others (bit 0) dec::Gen's step, or the 24-bit one
+// where that is not set up or a base is too large for it (bit 1).
 int launch_steps(mr_ctx *x, uint32_t classes, int steps)
 {
     const dec::Args A = dec_args(x->d, x->logm);
     for (int lm = dec::MIN_LM; lm <= dec::MAX_LM; lm++)
         if (classes >> lm & 1u) dec::launch_exp(lm, A, x->tab[lm], x->n, steps, x->st);
-    if (!(classes & 1u)) return 0;
     return dispatch_logm(x->logm, [&](auto lg) {
-        exp_kernel<decltype(lg)::value><<<x->n, THREADS, 0, x->st>>>(x->d, x->T, x->K, steps);
+        constexpr int LG = decltype(lg)::value;
+        if (classes & 1u) {
+            dec::launch_gen_exp(gen_args(x), x->gen_tw, x->n, steps, x->st);
+            gen_store_kernel<LG><<<x->n, THREADS, 0, x->st>>>(x->d, x->gen, x->gen_dig, x->gen.Lw + 2,
+                                                               x->gen_flag, nullptr, 0);
+        }
+        if (classes & 2u) exp_kernel<LG><<<x->n, THREADS, 0, x->st>>>(x->d, x->T, x->K, steps);
         return 0;
     });
 }
 
-// The classes in use when a round's bases are at most max_base.
+// The paths in use (launch_steps' bits) when a round's bases lie in [min_base,
+// max_base].
 uint32_t round_classes(const mr_ctx *x, uint32_t min_base, uint32_t max_base)
 {
-    if (min_base > (uint32_t)dec::MAX_BASE) return 1u;
-    return x->classes | (max_base > (uint32_t)dec::MAX_BASE ? 1u : 0u);
+    uint32_t c = 0;
+    if (min_base <= (uint32_t)dec::MAX_BASE) c = x->classes;
+    if (max_base > (uint32_t)dec::MAX_BASE) c |= 2u;
+    if ((c & 1u) && !x->gen.lm) c = (c & ~1u) | 2u;
+    return c;
 }
 
 // Rounds of every base in order over the whole context.  all_bases = false:
@@ -1944,6 +2090,12 @@ int arith_launch(mr_ctx *x, int op, const uint64_t *A, const uint64_t *B, int ld
     MR_CHECK(hipSetDevice(x->device));
     const int rc = dispatch_logm(x->logm, [&](auto lg) {
         constexpr int LG = decltype(lg)::value;
+        if (x->gen.lm && (op == AR_MUL || op == AR_SQ)) {
+            dec::launch_gen_mul(gen_args(x), x->gen_tw, x->n, A, op == AR_MUL ? B : nullptr, ld, st);
+            gen_store_kernel<LG><<<x->n, THREADS, 0, st>>>(x->d, x->gen, x->gen_dig, x->gen.Lw + 2, x->gen_flag,
+                                                            out, ld);
+            return 0;
+        }
         arith_kernel<LG><<<x->n, THREADS, 0, st>>>(x->d, x->T, x->K, op, A, B, ld, out, flag, r2);
         return 0;
     });

@@ -71,6 +71,70 @@ static void run(const Form &f, double *dig, const double *mul, int steps)
     const int off = f.mode == TOP || !steps ? 0 : f.Lw;
     for (int i = 0; i < f.Lw; i++) dig[i] = X[pd(off + i)];
 }
+// mul x y R^-1 mod N (y == nullptr: x^2) in base 2^43, all operands as Lw
+// balanced digits; np: N' = -N^-1 mod R.
+template <int LM>
+static void run_gen(int Lw, const double *N, const double *np, const double *x, const double *y, double mul,
+                    double *out)
+{
+    using g = G<LM>;
+    std::vector<double> X(lds_words<LM>(), 1e300), bnd(3 * (g::THREADS / 64) + 3), tab(4 * tab_size<LM>());
+    std::vector<double> tr[3], park(3 * g::M + 4);
+    for (auto &t : tr) t.resize(2 * g::M);
+    build_tables(LM, tab.data());
+    std::barrier<> blk(g::THREADS);
+    std::vector<std::unique_ptr<std::barrier<>>> wv;
+    for (int w = 0; w < g::THREADS / 64; w++) wv.emplace_back(new std::barrier<>(64));
+    g_block = &blk;
+    g_wave = &wv;
+    std::vector<std::thread> th;
+    for (int t = 0; t < g::THREADS; t++)
+        th.emplace_back([&, t] {
+            t_id = t;
+            auto load = [&](const double *v) {
+                for (int i = t; i < Lw; i += g::THREADS) X[pd(i)] = v[i];
+                sync_waves();
+            };
+            const double *src[3] = {N, np, y};
+            for (int k = 0; k < (y ? 3 : 2); k++) {
+                load(src[k]);
+                transform<LM>(X.data(), Lw, tab.data(), tr[k].data());
+                sync_waves();
+            }
+            Twid<LM> h[hoisted<LM>() ? 2 : 1];
+            for (int i = 0; i < (hoisted<LM>() ? 2 : 0); i++)
+                h[i].load(tab.data() + (2 * (t / g::TP) + i) * tab_size<LM>(), t & (g::TP - 1));
+            load(x);
+            mont_step<LM>(X.data(), bnd.data(), prime_of(t / g::TP), Lw, tab.data(), 0, mul, h,
+                          y ? tr[2].data() : nullptr, tr[1].data(), tr[0].data(), park.data());
+        });
+    for (auto &x2 : th) x2.join();
+    for (int i = 0; i < Lw; i++) out[i] = X[pd(Lw + i)];
+}
+extern "C" int gen_shape(int L, int *lw, int *sh)
+{
+    const Gen g = gen_of(L);
+    *lw = g.Lw;
+    *sh = g.sh;
+    return g.lm;
+}
+extern "C" double gen_digit(const uint32_t *v, int n, int sh, int i) { return gen_limb(v, n, sh, i); }
+extern "C" int gen_mont(int lm, int Lw, const double *N, const double *np, const double *x, const double *y,
+                        double mul, double *out)
+{
+    switch (lm) {
+    case 7: run_gen<7>(Lw, N, np, x, y, mul, out); break;
+    case 8: run_gen<8>(Lw, N, np, x, y, mul, out); break;
+    case 9: run_gen<9>(Lw, N, np, x, y, mul, out); break;
+    case 10: run_gen<10>(Lw, N, np, x, y, mul, out); break;
+    case 11: run_gen<11>(Lw, N, np, x, y, mul, out); break;
+    case 12: run_gen<12>(Lw, N, np, x, y, mul, out); break;
+    case 13: run_gen<13>(Lw, N, np, x, y, mul, out); break;
+    case 14: run_gen<14>(Lw, N, np, x, y, mul, out); break;
+    default: return 0;
+    }
+    return 1;
+}
 extern "C" int dec_choose(long long D, long long lo, long long hi, int *mode)
 {
     const Choice c = choose(D, lo, hi);

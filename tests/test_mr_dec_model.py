@@ -30,6 +30,11 @@ def model(tmp_path_factory):
     L.dec_choose.argtypes = [C.c_longlong, C.c_longlong, C.c_longlong, C.POINTER(C.c_int)]
     L.dec_square.argtypes = [C.POINTER(C.c_longlong), C.c_int, C.c_longlong, C.c_int, C.c_int,
                              C.POINTER(C.c_double), C.POINTER(C.c_double), C.c_int]
+    dp = C.POINTER(C.c_double)
+    L.gen_shape.argtypes = [C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)]
+    L.gen_digit.argtypes = [C.POINTER(C.c_uint32), C.c_int, C.c_int, C.c_int]
+    L.gen_digit.restype = C.c_double
+    L.gen_mont.argtypes = [C.c_int, C.c_int, dp, dp, dp, dp, C.c_double, dp]
     return L
 
 
@@ -114,3 +119,54 @@ def test_what_is_not_taken(model):
     assert model.dec_choose(5000, 100, 4999, C.byref(m)) == 10 and m.value == DENSE
     assert model.dec_choose(5000, 12, 4980, C.byref(m)) == 0
     assert model.dec_choose(120000, 100, 60000, C.byref(m)) == 0
+
+
+def balanced_digits(x, n):
+    out = (C.c_double * n)()
+    for i in range(n):
+        d = x & ((1 << 43) - 1)
+        if d >= 1 << 42:
+            d -= 1 << 43
+        out[i] = d
+        x = (x - d) >> 43
+    assert x == 0
+    return out
+
+
+@pytest.mark.parametrize("L", [4, 64, 102, 103, 207, 210, 440, 900, 1828, 1829, 6921, 13842])
+def test_any_modulus_step(model, L):
+    """mul x y R^-1 mod N in base 2^43 for random moduli of L 24-bit limbs,
+    and the largest (all digits ones); squares and products, mul up to 511."""
+    rng = random.Random(L)
+    lw, sh = C.c_int(), C.c_int()
+    lm = model.gen_shape(L, C.byref(lw), C.byref(sh))
+    Lw, sh = lw.value, sh.value
+    assert lm and 43 * Lw == 24 * L + sh and sh >= 16 and 2 * Lw + 4 <= 1 << lm
+    R = 1 << (43 * Lw)
+    for big in ([False, True] if L < 2000 else [True]):
+        N = (1 << (24 * L - 1)) - 1 if big else rng.getrandbits(24 * L - 1) | 1 | (1 << (24 * L - 2))
+        np_ = balanced_digits((-pow(N, -1, R)) % R, Lw + 1)
+        assert abs(np_[Lw]) <= 1
+        for mul, with_y in ([(1, True), (511, False)] if L < 2000 else [(511, False)]):
+            x, y = rng.randrange(N), N - 1 if big else rng.randrange(N)
+            out = (C.c_double * Lw)()
+            assert model.gen_mont(lm, Lw, balanced_digits(N, Lw), np_, balanced_digits(x, Lw),
+                                  balanced_digits(y, Lw) if with_y else None, mul, out)
+            z = sum(int(v) << (43 * i) for i, v in enumerate(out))
+            assert (z * R - mul * x * (y if with_y else x)) % N == 0
+            assert abs(z) <= N and max(abs(v) for v in out) <= 2.0 ** 42 + 2 ** 12
+
+
+def test_digits_of_24_bit_limbs(model):
+    """Limb i of 2^sh times a number of 24-bit limbs: the balanced digits sum to
+    it, for every shift a step uses."""
+    rng = random.Random(5)
+    for L in (4, 5, 43, 86):
+        for sh in range(0, 60):
+            v = [rng.choice([0, (1 << 24) - 1, rng.getrandbits(24)]) for _ in range(L)]
+            v[-1] &= (1 << 22) - 1
+            arr = (C.c_uint32 * L)(*v)
+            n = (24 * L + sh + 42) // 43 + 1
+            x = sum(int(model.gen_digit(arr, L, sh, i)) << (43 * i) for i in range(n))
+            assert x == sum(w << (24 * i) for i, w in enumerate(v)) << sh, (L, sh)
+            assert all(abs(model.gen_digit(arr, L, sh, i)) <= 1 << 42 for i in range(n))
