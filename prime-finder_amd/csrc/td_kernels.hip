@@ -328,8 +328,8 @@ void td_rows_kernel(const uint32_t *__restrict__ tbl, const uint32_t *__restrict
 
     const uint32_t count = min(ctrl[CT_SMALL_COUNT], TD_SMALL_CAP);
     const uint32_t row = threadIdx.x % TD_ROWS;
-    const uint32_t slot = threadIdx.x / TD_ROWS;
-    constexpr uint32_t nslots = TD_BLOCK / TD_ROWS;
+    const uint32_t slot = blockIdx.y * (TD_BLOCK / TD_ROWS) + threadIdx.x / TD_ROWS;
+    const uint32_t nslots = gridDim.y * (TD_BLOCK / TD_ROWS);
     const uint32_t k = k0 + row;
     if (k <= K) {
         const int lk = td_ndigits(k);
@@ -449,7 +449,7 @@ void td_fill_table_kernel(uint32_t J, uint32_t *__restrict__ tab)
 // (row, work item) instead of (row, prime), so the many marks of the
 // smallest primes are shared by many lanes.  rdec is the DJ-digit decode
 // table.  Falls back to whole primes if the item list overflowed.  The
-// fill primes present in the list (ctrl[CT_FILL]) are marked first, a word
+// band's items are strided over its gridDim.y workgroups.  The fill primes present in the list (ctrl[CT_FILL]) are marked first, a word
 // at a time: per row and fill prime the N condition's hits are the j of one
 // class mod p (j = u + 1 + t p) and the rev condition's the j whose R(j) is
 // of one class, so the row's words are ORs of the table's class masks,
@@ -469,9 +469,10 @@ void td_rows_bal_kernel(const uint32_t *__restrict__ tbl, const uint32_t *__rest
     const uint32_t w0 = ((k0 - 1u) * J) >> 5;
     const uint32_t nw = ((k_last * J - 1u) >> 5) - w0 + 1u;
     for (uint32_t w = threadIdx.x; w < nw; w += TD_BLOCK) lds[w] = 0u;
-    const uint32_t fill = ctrl[CT_FILL];
+    // one of the band's gridDim.y workgroups marks the fill primes
+    const uint32_t fill = blockIdx.y ? 0u : ctrl[CT_FILL];
     const uint32_t qw = (J + 31u) >> 5;
-    if (threadIdx.x < TD_ROWS * TD_NFILL) {
+    if (fill && threadIdx.x < TD_ROWS * TD_NFILL) {
         const uint32_t r = threadIdx.x / TD_NFILL, f = threadIdx.x - r * TD_NFILL;
         const uint32_t kk = k0 + r;
         uint32_t at_n = NONE, at_r = NONE;
@@ -523,8 +524,8 @@ void td_rows_bal_kernel(const uint32_t *__restrict__ tbl, const uint32_t *__rest
     }
 
     const uint32_t row = threadIdx.x % TD_ROWS;
-    const uint32_t slot = threadIdx.x / TD_ROWS;
-    constexpr uint32_t nslots = TD_BLOCK / TD_ROWS;
+    const uint32_t slot = blockIdx.y * (TD_BLOCK / TD_ROWS) + threadIdx.x / TD_ROWS;
+    const uint32_t nslots = gridDim.y * (TD_BLOCK / TD_ROWS);
     const uint32_t k = k0 + row;
     if (k <= K) {
         const int lk = td_ndigits(k);
@@ -1122,12 +1123,26 @@ int td_scratch(TdScratch **out)
     return 0;
 }
 
+// Workgroups per row band (gridDim.y of the row kernels): they share the
+// band's work items and OR their LDS copies of the band into the bitmap.
+// A lane's items form a serial chain of dependent loads, so few bands leave
+// the chip idle behind it: with one workgroup each the kernel took 131 us at
+// 256 x 256 (64 bands) and 180 at 333 x 777 (84 bands), against 17 and 132
+// here; 1024 bands (4096 x 4096) gain 6% from a second one and lose from a
+// fourth.  Above 16 the clearing and the merging of the band cost what the
+// shorter chains give.
+uint32_t td_row_split(uint32_t bands)
+{
+    return std::max(1u, std::min(16u, 2048u / bands));
+}
+
 template <int DJ>
 void td_launch_rest(const uint32_t *d_primes, uint32_t n, long long a, long long b,
                     long long c, uint32_t K, uint32_t J, uint32_t *d_bits,
                     const TdScratch &s, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1)
 {
-    const uint32_t row_groups = (K + TD_ROWS - 1u) / TD_ROWS;
+    const dim3 row_groups((K + TD_ROWS - 1u) / TD_ROWS,
+                          td_row_split((K + TD_ROWS - 1u) / TD_ROWS));
     const size_t lds = ((size_t)TD_ROWS * J / 32u + 2u) * sizeof(uint32_t);
     // The row kernel and the mid-range k loop (both latency-bound: few waves,
     // long dependent chains, frequent hit paths) run in turn on the
