@@ -465,6 +465,42 @@ PF_DEC_HD void make_form(const int64_t *terms, int nterm, int64_t D, int lm, int
     if (f.gap < 1) f.lm = 0;
 }
 
+// Group k >= 1 of Q as limbs: lo at limb E, hi at limb E + 1.
+struct Share { int32_t E; int64_t lo, hi; };
+PF_DEC_HD Share share_of(const Form &f, int k)
+{
+    const Term &t = f.t[k];
+    const int64_t x = (int64_t)DIGITS * (t.E + (f.mode == TOP ? f.Lw : 0)) + t.s - f.z;
+    const int64_t c = (int64_t)(t.c < 0.0 ? -t.c : t.c);
+    int64_t ts = 1;
+    for (int i = 0; i < (int)(x % DIGITS); i++) ts *= 10;
+    const int64_t tc = 10000000000000ll / ts;
+    return {(int32_t)(x / DIGITS), c % tc * ts, c / tc};
+}
+
+// Whether the digits v[0 .. Lw) of a number are m N + add (m 0 or 1; sh: the
+// shares of groups 1 .. nt - 1): their difference is carried up from the lowest
+// limb, where nearly every number that differs ends it.
+template <class V>
+PF_DEC_HD bool equals(const V *v, const Form &f, const Share *sh, int m, int add)
+{
+    const int64_t Bi = 10000000000000ll;
+    const int ED = f.D / DIGITS;
+    int64_t c = m - add, top = m;               // N = 10^D - 1 - groups
+    for (int i = 0; i < f.D % DIGITS; i++) top *= 10;
+    for (int i = 0; i < f.Lw + 2; i++) {
+        c += i < f.Lw ? (int64_t)v[i] : 0;
+        if (m) {
+            c -= i == ED ? top : 0;
+            for (int k = 1; k < f.nt; k++)
+                c += (i == sh[k].E ? sh[k].lo : 0) + (i == sh[k].E + 1 ? sh[k].hi : 0);
+        }
+        if (c % Bi) return false;
+        c /= Bi;
+    }
+    return c == 0;
+}
+
 // Where T waits during a DENSE squaring: in the LDS, behind the transforms (and
 // the zero word), where it fits; its limbs come back a barrier later instead of
 // a trip to memory.

@@ -561,6 +561,7 @@ __device__ __forceinline__ void mul_small_vec(uint32_t (&x)[C], uint32_t s, Scra
 {
     const int t = tid_();
     uint64_t acc = t ? 0ull : add;
+    asm("" : "+v"(s));      // a constant below 2^24 would lose the limbs' masks (from_digits)
 #pragma unroll
     for (int i = 0; i < C; i++) {
         acc += (uint64_t)x[i] * s;
@@ -627,15 +628,37 @@ __device__ __forceinline__ void pow5(Smem<LOGM> &sm, const Twiddles &T, const Co
 }
 
 // r <- sum of digits[i] 10^(13 i) over i < n (digits in LDS, each below 2^46).
+// Horner, one digit a step.  A thread's run of limbs is multiplied by 10^4, then
+// by 10^9, and what leaves it goes to the next thread's two lowest limbs, which
+// stay unreduced (below 2^25) until the end: two short barriers a digit, where
+// products with carries resolved throughout took 1.85 us.  (10^9 needs more than
+// 24 bits on purpose: a product of a masked 24-bit value and a 24-bit constant
+// plus a 64-bit addend is compiled here without the mask, and wrong.)
 template <int C>
 __device__ __forceinline__ void from_digits(uint32_t (&r)[C], const uint64_t *digits, int n, Scratch &sc)
 {
+    static_assert(C >= 2, "the lowest two limbs take the carry");
+    const int t = tid_();
 #pragma unroll
     for (int i = 0; i < C; i++) r[i] = 0u;
-    for (int i = n - 1; i >= 0; i--) {          // 10^13 = 10^6 10^7
-        mul_small_vec<C>(r, 1000000u, sc);
-        mul_small_vec<C>(r, 10000000u, sc, digits[i]);
+    for (int i = n - 1; i >= 0; i--) {
+        uint64_t a = 0, b = t ? 0ull : digits[i];
+#pragma unroll
+        for (int j = 0; j < C; j++) {
+            a += (uint64_t)r[j] * 10000u;
+            b += (a & LIMB_MASK) * 1000000000u;
+            r[j] = (uint32_t)b & LIMB_MASK;
+            a >>= LIMB_BITS;
+            b >>= LIMB_BITS;
+        }
+        sc.carry[t] = a * 1000000000u + b;      // about r[C - 1] 10^13 / 2^24, below 2^44
+        lds_barrier();
+        const uint64_t in = t ? sc.carry[t - 1] : 0ull;
+        lds_barrier();
+        r[0] += (uint32_t)in & LIMB_MASK;
+        r[1] += (uint32_t)(in >> LIMB_BITS);    // < 2^24 + 2^20
     }
+    mul_small_vec<C>(r, 1u, sc);
 }
 
 // The slot's canonical digits (left at scr by dec::launch_norm) as a number
@@ -1038,23 +1061,21 @@ __global__ __launch_bounds__(THREADS) void round_end_kernel(Dev D, Twiddles T, C
     const uint32_t *one = D.one + (size_t)c * D.stride;
     const uint32_t *nm1 = D.nm1 + (size_t)c * D.stride;
     uint32_t r[C];
-    if (D.path && D.path[c]) {      // digits: plain residue, s = 1
-        dec_value<LOGM>(sm, D, c, r);
-        if (out) store_vec<C>(r, out + (size_t)c * out_stride, L, 0);
-        uint32_t n[C];
-        load_vec<C>(n, D.N + (size_t)c * D.stride, L, 0);
-        bool no1 = false, nom = false, no0 = false;
-#pragma unroll
-        for (int i = 0; i < C; i++) {
-            const uint32_t u = threadIdx.x == 0 && i == 0 ? 1u : 0u;
-            no1 |= r[i] != u;
-            nom |= r[i] != n[i] - u;                            // N is odd
-            no0 |= r[i] != 0u;
+    if (D.path && D.path[c]) {      // digits in [0, 1.1 N): plain residue, s = 1
+        // compared as they are (converting them to 24-bit limbs for it took 1.28
+        // ms at 9000 digits)
+        const dec::Form &f = D.form[c];
+        dec::Share *sh = (dec::Share *)sm.X;
+        if ((int)threadIdx.x < f.nt && threadIdx.x) sh[threadIdx.x] = dec::share_of(f, threadIdx.x);
+        __syncthreads();
+        const int t = threadIdx.x;              // 0, 1, N - 1, N, N + 1
+        const bool pass = t < 5 && dec::equals((const double *)(D.scr + (size_t)c * 2 * G<LOGM>::M), f, sh,
+                                               t >= 2, t < 2 ? t : t - 3);
+        if (!block_any(pass, sm.sc) && t == 0) D.alive[c] = 0;
+        if (out) {
+            dec_value<LOGM>(sm, D, c, r);
+            store_vec<C>(r, out + (size_t)c * out_stride, L, 0);
         }
-        no1 = block_any(no1, sm.sc);
-        nom = block_any(nom, sm.sc);
-        no0 = block_any(no0, sm.sc);
-        if (threadIdx.x == 0 && no1 && nom && no0) D.alive[c] = 0;
         return;
     }
     load_vec<C>(r, D.res + (size_t)c * D.stride, L, L);
@@ -1235,39 +1256,52 @@ __global__ __launch_bounds__(THREADS) void dec_load_kernel(Dev D, Twiddles T, Co
         }
     store_vec<C>(r, scr, L, L);
     __syncthreads();
-    float *car = (float *)sm.X;                 // [2][Lw + 1] carries, |q| <= 2^23
+    // Balanced digits by Horner from the top, 40 bits a step, a run of ND digits
+    // per thread: the carries within a run stay in registers, one per run passes
+    // through the LDS, and waves above the value's length so far only keep the
+    // barrier.  |q| <= 2^40 leaves digits below B / 2 + 2^40; the last step (no
+    // shift) brings them to B / 2 + 1.  (24 bits a step with neighbouring digits
+    // in neighbouring lanes, every carry through the LDS: 16.5 ms at 50 000
+    // digits.)
+    constexpr int W = 40;
+    double *car = (double *)sm.sc.carry, *limb = (double *)sm.X;
+    const int steps = (LIMB_BITS * L + W - 1) / W;
+    for (int i = t; i < steps; i += THREADS) {
+        const int at = i * W / LIMB_BITS, sh = i * W % LIMB_BITS;
+        uint64_t v = scr[at];
+        if (at + 1 < L) v |= (uint64_t)scr[at + 1] << LIMB_BITS;
+        uint64_t hi = at + 2 < L ? scr[at + 2] : 0u;
+        limb[i] = (double)(((v >> sh) | hi << (2 * LIMB_BITS - sh)) & ((1ull << W) - 1));
+    }
     double x[ND];
 #pragma unroll
     for (int n = 0; n < ND; n++) x[n] = 0.0;
-    for (int i = threadIdx.x; i < 2 * Lw + 2; i += THREADS) car[i] = 0.0f;
     __syncthreads();
-    uint32_t limb = scr[L - 1];
-    for (int i = L - 1; i >= 0; i--) {
-        float *in = car + (i & 1) * (Lw + 1);
-        if (threadIdx.x == 0) in[0] = (float)limb;
-        limb = i ? scr[i - 1] : 0u;
+    const int k0 = t * ND, kw = (t & ~63) * ND;
+    double next = limb[steps - 1];
+    for (int i = steps - 1; i >= -1; i--) {
+        const double up = i >= 0 ? (double)(1ull << W) : 1.0, in0 = i >= 0 ? next : 0.0;
+        next = i > 0 ? limb[i - 1] : 0.0;
+        double q = 0.0;
+        // (the value has at most (steps - i) W bits; B > 2^43)
+        if (kw * 43 <= (steps - i) * W) {
 #pragma unroll
-        for (int n = 0; n < ND; n++) {
-            const int k = t + n * THREADS;
-            if (k < Lw) {
-                // (the top limb keeps its whole value: below B, maybe above B/2)
-                const double h = x[n] * 16777216.0, q = k + 1 < Lw ? __builtin_rint(h * dec::IB) : 0.0;
-                x[n] = __builtin_fma(-q, dec::B, h);
-                in[k + 1] = (float)q;
+            for (int n = 0; n < ND; n++) {
+                const double h = x[n] * up;
+                const double o = q;
+                // (the top digit keeps its whole value: below B, maybe above B/2)
+                q = k0 + n + 1 < Lw ? __builtin_rint(h * dec::IB) : 0.0;
+                x[n] = __builtin_fma(-q, dec::B, h) + o;
             }
         }
+        car[t] = q;
         lds_barrier();
-#pragma unroll
-        for (int n = 0; n < ND; n++) {
-            const int k = t + n * THREADS;
-            if (k < Lw) x[n] += (double)in[k];
-        }
+        x[0] += t ? car[t - 1] : in0;
+        lds_barrier();
     }
 #pragma unroll
-    for (int n = 0; n < ND; n++) {
-        const int k = t + n * THREADS;
-        if (k < Lw) D.dig[(size_t)c * D.dstride + k] = x[n];
-    }
+    for (int n = 0; n < ND; n++)
+        if (k0 + n < Lw) D.dig[(size_t)c * D.dstride + k0 + n] = x[n];
 }
 
 // R mod N of dec::Gen's step, 2^sh times the 24-bit form's, at the upper half

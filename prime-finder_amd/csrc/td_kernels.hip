@@ -1127,7 +1127,7 @@ int td_scratch(TdScratch **out)
 // band's work items and OR their LDS copies of the band into the bitmap.
 // A lane's items form a serial chain of dependent loads, so few bands leave
 // the chip idle behind it: with one workgroup each the kernel took 131 us at
-// 256 x 256 (64 bands) and 180 at 333 x 777 (84 bands), against 17 and 132
+// 256 x 256 (64 bands) and 180 at 1500 x 777 (375 bands), against 17 and 132
 // here; 1024 bands (4096 x 4096) gain 6% from a second one and lose from a
 // fourth.  Above 16 the clearing and the merging of the band cost what the
 // shorter chains give.

@@ -141,6 +141,17 @@ extern "C" int dec_choose(long long D, long long lo, long long hi, int *mode)
     *mode = c.mode;
     return c.lm;
 }
+// 1 when the digits are m N + add
+extern "C" int dec_equals(const long long *terms, int nterm, long long D, int lm, int mode, const double *dig,
+                          int m, int add)
+{
+    Form f;
+    std::vector<int64_t> t(terms, terms + 2 * nterm);
+    make_form(t.data(), nterm, D, lm, mode, f);
+    Share sh[MAX_TERMS];
+    for (int k = 1; k < f.nt; k++) sh[k] = share_of(f, k);
+    return equals(dig, f, sh, m, add);
+}
 // terms: nterm (coef, exp) pairs; dig: room for 8192; returns Lw (0: not handled)
 extern "C" int dec_square(const long long *terms, int nterm, long long D, int lm, int mode, double *dig,
                           const double *mul, int steps)

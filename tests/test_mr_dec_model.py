@@ -108,6 +108,31 @@ def test_square_step(model, case, kind):
     assert 10 * abs(y) <= 6 * (B ** Lw if mode.value == TOP else N)
 
 
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}-{c[1]}-{c[2]}{'r' if c[5] else ''}")
+def test_verdict_on_digits(model, case):
+    """The digits of 0, 1, N - 1, N, N + 1 are told from each other and from
+    numbers that differ from them in one digit."""
+    D, b, c, k, j, rev, _ = case
+    terms, lo, hi = terms_of(D, b, c, k, j, rev)
+    N = sum(q * 10 ** e for q, e in terms)
+    mode = C.c_int()
+    lm = model.dec_choose(D, lo, hi, C.byref(mode))
+    Lw = (D + (0 if mode.value == TOP else 8) + 12) // 13
+    flat = [v for t in terms for v in t]
+    arr = (C.c_longlong * len(flat))(*flat)
+    wanted = [(0, 0), (0, 1), (1, -1), (1, 0), (1, 1)]
+    for m, add in wanted:
+        v = m * N + add
+        for x in (v, v + B ** (Lw // 2), v + 10 ** (D - 1), v ^ 2):
+            if x >= B ** Lw:
+                continue
+            dig, y = (C.c_double * Lw)(), x
+            for i in range(Lw):
+                y, dig[i] = divmod(y, B)
+            got = [bool(model.dec_equals(arr, len(terms), D, lm, mode.value, dig, p, q)) for p, q in wanted]
+            assert got == [x == p * N + q for p, q in wanted], (m, add)
+
+
 def test_what_is_not_taken(model):
     """Short numbers, terms that leave no gap, and a least exponent below 2
     (N - 1 may be divisible by 4) stay with the Montgomery step."""
