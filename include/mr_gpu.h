@@ -180,7 +180,9 @@ mr_sched_t *mr_sched_create(const uint32_t *bases, int n_bases, int device,
 /* Device bytes one job of a candidate with `bits` bits occupies while
  * admitted (its slot: N, NTT(N), NTT(N'), residue, transform scratch), the
  * footprint admission counts against hbm_budget; -1 beyond this build's
- * sizes. */
+ * sizes.  Where the budget holds max_active such slots of every size and as
+ * much again, slots are larger (residues in base 10^13 beside them, which the
+ * squarings of search-form candidates run on) and admission counts that. */
 int64_t mr_sched_job_bytes(int64_t bits);
 /* Queue n candidates (validated first; -1 and nothing queued if any cannot
  * be formed or is too large). */

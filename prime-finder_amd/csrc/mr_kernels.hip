@@ -1635,6 +1635,25 @@ int ctx_alloc(mr_ctx *x, void **p, size_t bytes)
     return 0;
 }
 
+// Arrays that only a faster path needs: false without memory for all of them,
+// with none of them kept (the context then runs without that path).
+bool ctx_try_alloc(mr_ctx *x, std::initializer_list<std::pair<void **, size_t>> want)
+{
+    const size_t had = x->allocs.size();
+    for (const auto &w : want) {
+        if (hipMalloc(w.first, w.second) == hipSuccess) {
+            x->allocs.push_back(*w.first);
+            if (hipMemsetAsync(*w.first, 0, w.second, x->st) == hipSuccess) continue;
+        }
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(x->st);
+        for (; x->allocs.size() > had; x->allocs.pop_back()) (void)hipFree(x->allocs.back());
+        for (const auto &v : want) *v.first = nullptr;
+        return false;
+    }
+    return true;
+}
+
 constexpr int TMAX = 24;       // sparse decimal terms per candidate
 
 // Limbs and log2 transform length for numbers of at most `bits` bits:
@@ -1662,7 +1681,8 @@ dec::Args dec_args(const Dev &d, int logm)
 }
 
 // Geometry and device arrays for numbers of at most `bits` bits; with_dec:
-// also the base-10^13 path's, dense_lm: up to which class with N' (0: none).
+// also the base-10^13 path's where memory allows (d.form is set then), dense_lm:
+// up to which class with N' (0: none).
 int ctx_alloc_all(mr_ctx *x, long bits, int min_logm, bool with_dec = false, int dense_lm = 0)
 {
     int L, logm;
@@ -1706,13 +1726,13 @@ int ctx_alloc_all(mr_ctx *x, long bits, int min_logm, bool with_dec = false, int
     MR_ALLOC(done, uint8_t, n);
     if (with_dec) {
         d.dstride = dec_limbs(bits);
-        MR_ALLOC(form, dec::Form, n);
-        MR_ALLOC(path, int32_t, n);
-        MR_ALLOC(dig, double, n * d.dstride);
         d.tstride = dense_lm ? 2 << dense_lm : 0;
-        MR_ALLOC(decNt, double, dense_lm ? n * d.tstride : 1);
         d.pstride = 2 * d.dstride + (dec_limbs(bits) * 2 + 4 > 1 << 13 ? 3 << dec::MAX_LM >> 1 : 0);
-        MR_ALLOC(park, double, n * d.pstride);
+        (void)ctx_try_alloc(x, {{(void **)&d.form, n * sizeof(dec::Form)},
+                                {(void **)&d.path, n * sizeof(int32_t)},
+                                {(void **)&d.dig, n * d.dstride * sizeof(double)},
+                                {(void **)&d.decNt, (dense_lm ? n * d.tstride : 1) * sizeof(double)},
+                                {(void **)&d.park, n * d.pstride * sizeof(double)}});
     }
 #undef MR_ALLOC
     d.list = nullptr;
@@ -1760,11 +1780,11 @@ int gen_setup(mr_ctx *x)
     const size_t n = (size_t)x->n, M = (size_t)1 << g.lm;
     if (!(x->gen_tw = dec::tables(x->device, g.lm))) return -2;
     x->gen_pstride = 2 * g.Lw + 2 + (g.lm > 13 ? 3 << g.lm >> 1 : 0);
-    if (ctx_alloc(x, (void **)&x->gen_tab, n * 10 * M * sizeof(double)) != 0 ||
-        ctx_alloc(x, (void **)&x->gen_dig, n * (g.Lw + 2) * sizeof(double)) != 0 ||
-        ctx_alloc(x, (void **)&x->gen_park, n * x->gen_pstride * sizeof(double)) != 0 ||
-        ctx_alloc(x, (void **)&x->gen_flag, n * sizeof(int32_t)) != 0)
-        return -2;
+    if (!ctx_try_alloc(x, {{(void **)&x->gen_tab, n * 10 * M * sizeof(double)},
+                           {(void **)&x->gen_dig, n * (g.Lw + 2) * sizeof(double)},
+                           {(void **)&x->gen_park, n * x->gen_pstride * sizeof(double)},
+                           {(void **)&x->gen_flag, n * sizeof(int32_t)}}))
+        return 0;
     x->gen = g;
     x->d.gen = 1;
     (void)dispatch_logm(x->logm, [&](auto lg) {
@@ -2456,6 +2476,7 @@ extern "C" mr_ctx_t *mr_ctx_create_sparse(const mr_candidate_t *cands, int n_bat
     mr_ctx *x = ctx_new((int)((bits + 31) / 32), n_batch, device);
     if (!x) return nullptr;
     int rc = ctx_alloc_all(x, (long)x->n_words * 32, g_min_logm, true, dense ? 31 - __builtin_clz(dense) : 0);
+    if (rc == 0 && !x->d.form) { classes = 1u; dense = 0; }
     x->classes = classes;
     for (int lm = dec::MIN_LM; lm <= dec::MAX_LM && rc == 0; lm++)
         if (classes >> lm & 1u && !(x->tab[lm] = dec::tables(x->device, lm))) rc = -2;
@@ -2470,7 +2491,8 @@ extern "C" mr_ctx_t *mr_ctx_create_sparse(const mr_candidate_t *cands, int n_bat
     if (rc == 0)
         rc = dispatch_logm(x->logm, [&](auto lg) {
             constexpr int LG = decltype(lg)::value;
-            dec::launch_form(nullptr, x->n, dterms, TMAX, dchoice, x->d.form, x->d.err, x->st);
+            if (x->d.form)
+                dec::launch_form(nullptr, x->n, dterms, TMAX, dchoice, x->d.form, x->d.err, x->st);
             for (int lm = dec::MIN_LM; lm <= dec::MAX_LM; lm++)
                 if (dense >> lm & 1u) dec::launch_prepare(lm, dec_args(x->d, x->logm), x->tab[lm], x->n, x->st);
             build_kernel<LG><<<x->n, THREADS, 0, x->st>>>(x->d, x->T, x->K, dterms, TMAX, nullptr);
@@ -2575,16 +2597,18 @@ int dec_pool_lm(int logm)
 
 // Bytes of device memory per slot of a pool of transform length 2^logm
 // (the arrays of ctx_alloc_all).
-int64_t slot_bytes(int logm)
+int64_t slot_bytes(int logm, bool with_dec = false)
 {
     const int64_t M = 1ll << logm;
-    return 4 * (4 * M + 7 * M + (split_logm(logm) ? M + M / 2 : 0) + (half_logm(logm) ? M : 0)) + 32 +
-           (int64_t)sizeof(dec::Form) + 4 + 24 * dec_limbs(pool_bits(logm)) + 16 * (1ll << dec_pool_lm(logm)) +
+    const int64_t plain = 4 * (4 * M + 7 * M + (split_logm(logm) ? M + M / 2 : 0) + (half_logm(logm) ? M : 0)) + 32;
+    if (!with_dec) return plain;
+    return plain + (int64_t)sizeof(dec::Form) + 4 + 24 * dec_limbs(pool_bits(logm)) + 16 * (1ll << dec_pool_lm(logm)) +
            (dec_pool_lm(logm) > 13 ? 12ll << dec::MAX_LM : 0);
 }
 
 struct Pool {
     int logm = 0, n = 0;
+    int64_t per = 0;                // bytes of a slot
     int chunk = 0;                  // squaring steps per chunk (graph launch)
     mr_ctx *x = nullptr;            // x->st is the admin stream
     hipStream_t st_run = nullptr;
@@ -2677,7 +2701,13 @@ void pool_free(Pool *p)
 
 int pool_new(mr_sched *S, int logm, Pool **out)
 {
-    const int64_t per = slot_bytes(logm);
+    // The base-10^13 arrays about double a slot: pools have them where the budget
+    // holds every size's full pool with them, so that a tighter one still admits
+    // as many jobs at once as without them.
+    int64_t all = 0;
+    for (int lg = MIN_LOGM; lg <= MAX_LOGM; lg++) all += (int64_t)S->max_active * slot_bytes(lg, true);
+    const bool with_dec = all <= S->budget;
+    const int64_t per = slot_bytes(logm, with_dec);
     int64_t room = (S->budget - S->hbm) / per;
     int n = std::min(S->bucket_slots[logm] ? S->bucket_slots[logm] : S->pool_slots, S->max_active);
     if (room < n) n = (int)room;
@@ -2686,10 +2716,11 @@ int pool_new(mr_sched *S, int logm, Pool **out)
     if (!p) return -2;
     p->logm = logm;
     p->n = n;
+    p->per = per;
     p->chunk = S->bucket_chunk[logm] ? S->bucket_chunk[logm] : S->chunk;
     p->x = ctx_new(1, n, S->device);
     int rc = p->x ? 0 : -2;
-    if (rc == 0) rc = ctx_alloc_all(p->x, pool_bits(logm), logm, true, dec_pool_lm(logm));
+    if (rc == 0) rc = ctx_alloc_all(p->x, pool_bits(logm), logm, with_dec, dec_pool_lm(logm));
     if (rc == 0 && p->x->logm != logm) rc = -1;
     auto dev = [&](void **q, size_t b) { if (rc == 0 && ctx_alloc(p->x, q, b) != 0) rc = -2; };
     dev((void **)&p->d_list_adm, 4 * (size_t)n);
@@ -2742,7 +2773,7 @@ void reclaim_idle(mr_sched *S, int except)
         Pool *&p = S->pools[lg];
         if (!p || lg == except || p->busy_slots || p->run_busy || p->adm_busy) continue;
         if (S->qhead[lg] < S->queue[lg].size()) continue;      // its own jobs are waiting
-        S->hbm -= slot_bytes(lg) * p->n;
+        S->hbm -= p->per * p->n;
         pool_free(p);
         p = nullptr;
         S->reclaimed++;
@@ -2889,7 +2920,7 @@ int launch_admin(mr_sched *S, Pool *p)
     uint32_t dense = 0;     // classes with N' to prepare
     std::vector<int> &queue = S->queue[p->logm];
     size_t &qh = S->qhead[p->logm];
-    const int64_t per = slot_bytes(p->logm);
+    const int64_t per = p->per;
     // a job is admitted when a slot of its bucket is free, the active cap
     // allows, and its footprint (its slot's device state) fits the budget
     for (int c = 0; c < p->n && qh < queue.size() && S->active < S->max_active &&
@@ -2903,6 +2934,7 @@ int launch_admin(mr_sched *S, Pool *p)
                                 q.cand.which};
         n_dev += q.dev_list ? 1 : 0;
         p->h_Ls[i] = q.L;
+        if (!p->x->d.form) q.choice = dec::Choice{0, 0};
         p->h_choice[3 * i] = (int32_t)q.digits;
         p->h_choice[3 * i + 1] = q.choice.lm;
         p->h_choice[3 * i + 2] = q.choice.mode;
@@ -2947,8 +2979,9 @@ int launch_admin(mr_sched *S, Pool *p)
             MR_CHECK(hipGetLastError());
         }
         MR_CHECK(hipMemcpyAsync(p->d_choice, p->h_choice, 12 * (size_t)n_new, hipMemcpyHostToDevice, st));
-        dec::launch_form(p->d_list_adm + n_end, n_new, p->d_terms, TMAX, p->d_choice, p->x->d.form,
-                         p->x->d.err, st);
+        if (p->x->d.form)
+            dec::launch_form(p->d_list_adm + n_end, n_new, p->d_terms, TMAX, p->d_choice, p->x->d.form,
+                             p->x->d.err, st);
         Dev Dp = p->x->d;
         Dp.list = p->d_list_adm + n_end;
         for (int lm = dec::MIN_LM; lm <= dec::MAX_LM; lm++) {
@@ -2991,7 +3024,7 @@ int launch_admin(mr_sched *S, Pool *p)
         }
         MR_CHECK(hipMemcpyAsync(p->d_resume, p->h_resume, 12 * (size_t)n_res, hipMemcpyHostToDevice, st));
         resume_kernel<<<(n_res + 63) / 64, 64, 0, st>>>(p->x->d, p->d_resume, n_res, bases);
-        (void)dispatch_logm(p->logm, [&](auto lg) {
+        if (p->x->d.form) (void)dispatch_logm(p->logm, [&](auto lg) {
             dec_load_kernel<decltype(lg)::value><<<n_res, THREADS, 0, st>>>(p->x->d, T, K, p->d_resume);
             return 0;
         });
@@ -3025,7 +3058,7 @@ int admin_done(mr_sched *S, Pool *p)
             p->state[c] = SL_FREE;
             p->req[c] = -1;
             S->active--;
-            S->job_bytes -= slot_bytes(p->logm);
+            S->job_bytes -= p->per;
             p->busy_slots--;
         } else {
             p->state[c] = SL_RUN;

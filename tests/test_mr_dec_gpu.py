@@ -57,3 +57,26 @@ def test_classes_side_by_side_and_mixed_bases(gpu):
         want, wr, _ = gmp_sprp(gmp_build(*cd), b)
         assert r == wr and o == bool(want), (cd, b)
     ctx.close()
+
+
+def test_budget_of_one_slot_without_the_digits(gpu, tmp_path):
+    """A budget of exactly one slot of 24-bit arrays (8 000 digits: 2^12 points,
+    12 M words and 32 bytes) takes the job and decides it; a checkpoint from
+    such a scheduler continues in one whose budget has room for the digits, and
+    the other way round."""
+    slot = 4 * 12 * 4096 + 32
+    assert gpu.lib().mr_sched_job_bytes(int(8000 * 3.3219280948873623) + 2) == slot
+    cd = (8000, 2500, 300, 4001, 17, 0)
+    want = gmp_sprp(gmp_build(*cd), 2)[0]
+    for first, then in ((slot, 0), (0, slot)):
+        s = gpu.MrScheduler([2], hbm_budget=first)
+        s.submit([cd], tags=[5])
+        for _ in range(3):
+            s.pump()
+        s.checkpoint(tmp_path / "c")
+        assert s.stats().peak_job_bytes >= slot
+        s.close()
+        s = gpu.MrScheduler([2], hbm_budget=then)
+        s.restore(tmp_path / "c")
+        assert [(r.tag, bool(r.verdict), r.rounds) for r in s.run_all()] == [(5, bool(want), 1)]
+        s.close()
