@@ -156,7 +156,11 @@ __global__ __launch_bounds__(G<LM>::THREADS) void norm_kernel(Args A)
     const int off = f.mode == TOP ? 0 : Lw;
     Terms u;
     load_terms(u, f);
-    if (f.mode != TOP) fold<LM>(X, G<LM>::XP, f, u, t);        // out of Montgomery form
+    if (f.mode == DENSE && f.gap < 1) {                        // out of Montgomery form
+        if (t == 0) solve(X, f, true);
+    } else if (f.mode != TOP) {
+        fold<LM>(X, G<LM>::XP, f, u, t);
+    }
     __syncthreads();
     if (t == 0) canonical(X, off, f);
     __syncthreads();

@@ -388,7 +388,7 @@ struct Form {
 // mod 4 (one squaring chain, s = 1); hi < D keeps Q below N/10.  Where the
 // fewer of the two modes' rounds would cost more than a second product
 // (dense_from rounds, measured), DENSE; its N' comes from BOTTOM's rounds, run
-// once.
+// once, or, where lo leaves them no gap, limb by limb (solve).
 constexpr int MAX_ROUNDS = 64, MIN_DIGITS = 40, MAX_BASE = 511;
 constexpr int dense_from(int lm) { return lm <= 8 ? 7 : lm <= 11 ? 8 : 10; }
 struct Choice { int32_t lm, mode; };
@@ -406,9 +406,9 @@ PF_DEC_HD Choice choose(int64_t D, int64_t lo, int64_t hi)
     const int64_t L = c.mode == TOP ? Lt : Lb;
     for (int lm = MIN_LM; lm <= MAX_LM && !c.lm; lm++)
         if ((1ll << lm) >= 2 * L + 4) c.lm = lm;
-    if (c.lm && gb >= 1 && (rt < rb ? rt : rb) >= dense_from(c.lm)) {
-        c.mode = DENSE;
-        if (2 * Lb + 4 > (1ll << c.lm)) c.lm = c.lm < MAX_LM ? c.lm + 1 : 0;
+    if (c.lm && (rt < rb ? rt : rb) >= dense_from(c.lm)) {
+        const int lm = 2 * Lb + 4 <= (1ll << c.lm) ? c.lm : c.lm < MAX_LM ? c.lm + 1 : 0;
+        if (lm || gb >= 1) c = {lm, DENSE};
     }
     return c;
 }
@@ -462,7 +462,7 @@ PF_DEC_HD void make_form(const int64_t *terms, int nterm, int64_t D, int lm, int
         put(at + f.z, mode == TOP ? (double)c : -(double)c);
     }
     f.gap = mode == TOP ? -f.omax - 2 : f.omin;
-    if (f.gap < 1) f.lm = 0;
+    if (f.gap < 1 && mode != DENSE) f.lm = 0;
 }
 
 // Group k >= 1 of Q as limbs: lo at limb E, hi at limb E + 1.
@@ -779,6 +779,63 @@ PF_DEC_FN double gather(double acc, double &car, const double *S, int s0, int s1
     return acc;
 }
 
+// v = q B + r, 0 <= r < B, for |v| < 2^92: the quotient estimated in FP64 (below
+// 2^49, off by a unit or two), r exact.
+PF_DEC_FN int64_t split(__int128 v, int64_t &r)
+{
+    const int64_t Bi = 10000000000000ll;
+    const double e = (double)(int64_t)(v >> 64) * 18446744073709551616.0 + (double)(uint64_t)v;
+    int64_t q = (int64_t)(e * IB);
+    v -= (__int128)q * Bi;
+    while (v < 0) { v += Bi; q--; }
+    while (v >= Bi) { v -= Bi; q++; }
+    r = (int64_t)v;
+    return q;
+}
+
+// T (limbs in LDS, padded; limbs from Lw up zero) -> m with T + m N = 0 mod R at
+// limbs [0, Lw), and, with high, (T + m N) / R at [Lw, 2 Lw): what BOTTOM's
+// rounds compute, limb by limb for terms that leave them no gap (digits of Q
+// below 10^13: a limb of m is the limb of the sum so far over the lowest limb of
+// 1 + Q's groups, a unit since every exponent is at least 2).  One thread; once
+// per candidate and per round, where up to MAX_ROUNDS fold rounds in every
+// squaring cost up to 13.7 us in class 8 against 4 (a batch of 300 numbers with one
+// such: 95 -> 64 ms).
+PF_DEC_FN void solve(double *T, const Form &f, bool high)
+{
+    const int64_t Bi = 10000000000000ll;
+    const int Lw = f.Lw, ED = f.D / DIGITS;
+    Share sh[MAX_TERMS];
+    int64_t u0 = 1, top = 1;
+    for (int i = 0; i < f.D % DIGITS; i++) top *= 10;
+    for (int k = 1; k < f.nt; k++) {
+        sh[k] = share_of(f, k);
+        if (sh[k].E == 0) u0 += sh[k].lo;
+    }
+    int64_t w = 1, x;                           // 1 / u0 mod B: 2, 4, 8, 16 digits
+    for (int n = 0; n < 3; n++) {
+        split((__int128)(u0 % Bi) * w, x);
+        split((__int128)w * (2 - x), w);
+    }
+    int64_t carry = 0;
+    for (int i = 0; i < (high ? 2 * Lw : Lw); i++) {
+        auto m = [&](int p) { return p >= 0 && p < Lw && p < i ? (int64_t)T[pd(p)] : (int64_t)0; };
+        __int128 v = (__int128)(int64_t)T[pd(i)] + carry + (__int128)top * m(i - ED);
+        for (int k = 1; k < f.nt; k++) v -= (__int128)sh[k].lo * m(i - sh[k].E) + (__int128)sh[k].hi * m(i - sh[k].E - 1);
+        int64_t d;
+        carry = split(v, d);
+        if (i < Lw) {
+            split((__int128)d * w, d);
+            if (d > Bi / 2) d -= Bi;
+            carry = split(v - (__int128)d * u0, x);
+        } else if (d > Bi / 2) {
+            d -= Bi;
+            carry++;
+        }
+        T[pd(i)] = (double)d;
+    }
+}
+
 // T (limbs in LDS, padded) -> the product reduced, at limbs [0, Lw) (TOP) or
 // [Lw, 2 Lw) (BOTTOM).  A round's targets lie outside its sources and span at
 // most Lw + 2 limbs.  T[zi] is zero.  (Cutting the targets into one window per
@@ -790,6 +847,12 @@ PF_DEC_FN void fold(double *T, int zi, const Form &f, const Terms &u, int t, dou
     constexpr int W = G<LM>::THREADS / 64, STEP = 62 * W, NI = (G<LM>::M / 2 + 1 + STEP) / STEP;
     const int lane = t & 63, wave = uniform(t >> 6);
     const int Lw = u.Lw, gap = u.gap;
+    if (rec && gap < 1) {
+        if (t == 0) solve(T, f, false);
+        sync_block<LM>();
+        for (int i = t; i < Lw; i += G<LM>::THREADS) rec[i] = T[pd(i)];
+        return;
+    }
     const bool top = u.mode == TOP;
     const int first = top ? Lw : 0, last = top ? 2 * Lw + 1 : Lw;
     for (int done = 0; first + done < last; done += gap) {

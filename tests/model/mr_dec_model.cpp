@@ -173,3 +173,15 @@ extern "C" int dec_square(const long long *terms, int nterm, long long D, int lm
     }
     return f.Lw;
 }
+// dig (2 Lw): x -> m and (x + m N) / R, limb by limb; returns Lw
+extern "C" int dec_solve(const long long *terms, int nterm, long long D, double *dig)
+{
+    Form f;
+    std::vector<int64_t> t(terms, terms + 2 * nterm);
+    make_form(t.data(), nterm, D, MAX_LM, DENSE, f);
+    std::vector<double> T(pd(2 * f.Lw) + 1);
+    for (int i = 0; i < 2 * f.Lw; i++) T[pd(i)] = dig[i];
+    solve(T.data(), f, true);
+    for (int i = 0; i < 2 * f.Lw; i++) dig[i] = T[pd(i)];
+    return f.Lw;
+}

@@ -80,3 +80,30 @@ def test_budget_of_one_slot_without_the_digits(gpu, tmp_path):
         s.restore(tmp_path / "c")
         assert [(r.tag, bool(r.verdict), r.rounds) for r in s.run_all()] == [(5, bool(want), 1)]
         s.close()
+
+
+@pytest.mark.parametrize("digits", [300, 780, 1600, 3000, 6600])
+def test_second_product_without_a_gap_below(gpu, tmp_path, digits):
+    """Least exponent below 13 and terms near the top (N' limb by limb): residues
+    against GMP, and a test continued from a checkpoint."""
+    a, gap = digits, digits // 20 + 26
+    cands = [(a, a - gap, 2, 4096, 4095, 0), (a, a - gap, 12, 1, 77, 0),
+             (a, a - 3 - len("4096"), gap, 4096, 4095, 1), (a, a - gap - 1, 7, 4095, 4096, 0)]
+    bases = [2, 511] if digits < 2000 else [2]
+    ctx = gpu.MrContext(candidates=cands)
+    _, res, passed = ctx.run(bases, all_bases=True, passes=True)
+    ctx.close()
+    for i, cd in enumerate(cands):
+        for j, base in enumerate(bases):
+            ok, r, _ = gmp_sprp(gmp_build(*cd), base)
+            assert (res[i][j], passed[i][j]) == (r, ok), (cd, base)
+    s = gpu.MrScheduler([2], chunk=64)
+    s.submit(cands, tags=[0, 1, 2, 3])
+    for _ in range(3):
+        s.pump()
+    s.checkpoint(tmp_path / "c")
+    s.close()
+    s = gpu.MrScheduler([2])
+    s.restore(tmp_path / "c")
+    assert [bool(r.verdict) for r in sorted(s.run_all(), key=lambda r: r.tag)] == [bool(p[0]) for p in passed]
+    s.close()

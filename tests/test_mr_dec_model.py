@@ -31,6 +31,7 @@ def model(tmp_path_factory):
     L.dec_square.argtypes = [C.POINTER(C.c_longlong), C.c_int, C.c_longlong, C.c_int, C.c_int,
                              C.POINTER(C.c_double), C.POINTER(C.c_double), C.c_int]
     dp = C.POINTER(C.c_double)
+    L.dec_solve.argtypes = [C.POINTER(C.c_longlong), C.c_int, C.c_longlong, dp]
     L.gen_shape.argtypes = [C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int)]
     L.gen_digit.argtypes = [C.POINTER(C.c_uint32), C.c_int, C.c_int, C.c_int]
     L.gen_digit.restype = C.c_double
@@ -131,6 +132,43 @@ def test_verdict_on_digits(model, case):
                 y, dig[i] = divmod(y, B)
             got = [bool(model.dec_equals(arr, len(terms), D, lm, mode.value, dig, p, q)) for p, q in wanted]
             assert got == [x == p * N + q for p, q in wanted], (m, add)
+
+
+LOW = [     # DENSE without a gap below: least exponent under 13, terms near the top
+    (300, 270, 5, 4096, 4095, False, 3), (780, 740, 2, 9999, 77, False, 2),
+    (1000, 930, 12, 4096, 1, False, 2), (1600, 1590, 100, 4096, 4095, True, 2),
+    (3000, 2870, 2, 1000000, 999999, False, 2), (3290, 3100, 3, 4096, 99, False, 1),
+    (6500, 6300, 7, 4096, 4095, False, 1), (26000, 25000, 9, 1, 4095, False, 1),
+]
+
+
+@pytest.mark.parametrize("kind", ["random", "largest", "ends"])
+@pytest.mark.parametrize("case", LOW, ids=lambda c: f"{c[0]}-{c[1]}-{c[2]}{'r' if c[5] else ''}")
+def test_second_product_without_a_gap_below(model, case, kind):
+    D, b, c, k, j, rev, _ = case
+    mode = C.c_int()
+    _, lo, hi = terms_of(D, b, c, k, j, rev)
+    assert lo < 13 and model.dec_choose(D, lo, hi, C.byref(mode)) >= 7 and mode.value == DENSE
+    test_square_step(model, case, kind)
+
+
+@pytest.mark.parametrize("case", LOW[:6], ids=lambda c: f"{c[0]}-{c[1]}-{c[2]}{'r' if c[5] else ''}")
+def test_reduction_limb_by_limb(model, case):
+    """x -> m and (x + m N) / R for x of random and of the largest digits."""
+    D, b, c, k, j, rev, _ = case
+    terms, _, _ = terms_of(D, b, c, k, j, rev)
+    N = sum(q * 10 ** e for q, e in terms)
+    Lw, rng = (D + 20) // 13, random.Random(D)
+    flat = [v for t in terms for v in t]
+    for pick in (lambda: rng.randint(-B // 2, B // 2), lambda: B // 2 + 65536, lambda: -B // 2 - 65536):
+        dig = (C.c_double * (2 * Lw))()
+        for i in range(Lw):
+            dig[i] = pick()
+        x = sum(int(dig[i]) * B ** i for i in range(Lw))
+        assert model.dec_solve((C.c_longlong * len(flat))(*flat), len(terms), D, dig) == Lw
+        m, y = (sum(int(dig[o + i]) * B ** i for i in range(Lw)) for o in (0, Lw))
+        assert x + m * N == y * B ** Lw
+        assert max(abs(v) for v in dig) <= B / 2
 
 
 def test_what_is_not_taken(model):
