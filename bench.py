@@ -66,9 +66,8 @@ INT32_VALU_PEAK_TOPS = 256 * 64 * 2.4e9 / 1e12      # 39.32 Tops/s (256 CUs, wav
 # readings: x2.0 and x1.0): 23.29 MB read (the prime list) + 478.65 MB
 # written (memory-side atomic ORs of the hits of the primes from 2^17).
 TD_TRAFFIC_BYTES = 23.29e6 + 478.65e6
-# Same for one batched squaring step of the 50 000-digit Miller-Rabin batch
-# (256 bigints, 2^14 transforms): 91.7 MB read + 14.4 MB written.
-MR_TRAFFIC_BYTES_PER_STEP = 91.7e6 + 14.4e6
+# FP64 instructions: 64 lanes per compute unit and clock, as INT32.
+FP64_VALU_PEAK_TOPS = 256 * 64 * 2.4e9 / 1e12
 
 
 def _load(name, path):
@@ -229,19 +228,18 @@ def cpu_baselines(budget_s: float) -> dict:
     return out
 
 
-def mr_ops_per_squaring(logm: int) -> int:
-    """INT32 VALU ops of one Montgomery squaring step on one candidate, by
-    the transform-count model T(M) = (M/2) log2(M) 12 per transform and
-    prime.  Per prime: r^2 and T_lo N' are products of M points (a forward
-    and an inverse transform each, the other operand precomputed), m N is a
-    wrapped product of M/2 points (its low half is known), so
-    ops = 2 (4 T(M) + 2 T(M/2) + 20 M) + 50 M, the 20 M and 50 M being the
-    pointwise products and the CRT/carry per coefficient, at this build's
-    transform length M = 2^logm (24-bit limbs: 2^14 at 50 000 digits)."""
-    M = 1 << logm
-    T = (M // 2) * logm * 12
-    Th = (M // 4) * (logm - 1) * 12
-    return 2 * (4 * T + 2 * Th + 20 * M) + 50 * M
+def mr_ops_per_squaring(digits: int) -> int:
+    """FP64 VALU instructions of one squaring step on one search-form
+    candidate (base 10^13, two 50-bit primes, M the power of two that holds
+    2 Lw + 4 limbs): a forward and an inverse transform of M points per prime
+    at 8 instructions per butterfly (a modular product is 6), 6 M per prime for
+    the pointwise squares and 30 M for the recombination and carries.  The fold
+    by the sparse terms, or the second product of a candidate whose terms leave
+    little room, comes on top and is not counted."""
+    lw = (digits + 8 + 12) // 13
+    lm = max(7, (2 * lw + 3).bit_length())
+    M = 1 << lm
+    return 2 * (2 * (M // 2) * lm * 8 + 6 * M) + 30 * M
 
 
 def mr_leg(pf, n_bits: int, digits: int = 50000) -> dict:
@@ -260,7 +258,7 @@ def mr_leg(pf, n_bits: int, digits: int = 50000) -> dict:
     bits = int(digits * 3.3219280948873623) - 1       # squarings per test (bits of d)
     step_s = ms / 1e3 / n_bits
     test_s = step_s * bits
-    ops = mr_ops_per_squaring(ctx.log_len) * len(cands)
+    ops = mr_ops_per_squaring(digits) * len(cands)
     achieved = ops / step_s / 1e12
     res = {"workload": f"256 bigints (128 N + 128 rev N) at {digits} digits, base 2",
            "limbs": ctx.limbs, "transform_len": 1 << ctx.log_len,
@@ -268,13 +266,9 @@ def mr_leg(pf, n_bits: int, digits: int = 50000) -> dict:
            "tests_per_hour_extrapolated": 3600.0 * len(cands) / test_s,
            "sample": f"{n_bits} of {bits} squaring steps timed (HIP events), scaled",
            "setup_s": setup_s,
-           "roofline": {"bound": "valu", "achieved": achieved, "peak": INT32_VALU_PEAK_TOPS,
-                        "unit": "Tops/s", "frac": achieved / INT32_VALU_PEAK_TOPS,
-                        "traffic": MR_TRAFFIC_BYTES_PER_STEP if ctx.log_len == 14 else None,
-                        "traffic_note": "HBM bytes per batched squaring step (rocprofv3 "
-                                        "FETCH_SIZE + WRITE_SIZE); algorithmic 50.3e6 "
-                                        "(NTT(N') and NTT(N) at M/2 points per bigint)",
-                        "kernel": f"exp_kernel<{ctx.log_len}>",
+           "roofline": {"bound": "valu", "achieved": achieved, "peak": FP64_VALU_PEAK_TOPS,
+                        "unit": "Tops/s", "frac": achieved / FP64_VALU_PEAK_TOPS,
+                        "kernel": "dec::exp_kernel",
                         "ops_per_squaring_step": ops}}
     ctx.close()
     return res
@@ -342,7 +336,7 @@ def mr_step_leg(pf, cands, n_bits: int, total_bits: int, label: str) -> dict:
     ctx.time_squarings(2, 64)
     step_s = ctx.time_squarings(2, n_bits) / 1e3 / n_bits
     logm = ctx.log_len
-    ops = mr_ops_per_squaring(logm) * len(cands)
+    ops = sum(mr_ops_per_squaring(c[0]) for c in cands)
     ctx.close()
     one = pf.MrContext(candidates=cands[:1])
     one.time_squarings(2, 64)
@@ -357,9 +351,9 @@ def mr_step_leg(pf, cands, n_bits: int, total_bits: int, label: str) -> dict:
             "sample": f"{n_bits} of {total_bits} squaring steps timed (HIP events), scaled",
             "plain_one_candidate": {"us_per_squaring": one_s * 1e6, "tests_per_hour": plain,
                                     "batched_over_plain": tph / plain},
-            "roofline": {"bound": "valu", "achieved": achieved, "peak": INT32_VALU_PEAK_TOPS,
-                         "unit": "Tops/s", "frac": achieved / INT32_VALU_PEAK_TOPS,
-                         "kernel": f"exp_kernel<{logm}>", "ops_per_squaring_step": ops}}
+            "roofline": {"bound": "valu", "achieved": achieved, "peak": FP64_VALU_PEAK_TOPS,
+                         "unit": "Tops/s", "frac": achieved / FP64_VALU_PEAK_TOPS,
+                         "kernel": "dec::exp_kernel", "ops_per_squaring_step": ops}}
 
 
 def mr_cpu_baseline(cands, budget_s: float = 15.0, sample_bits: int = 4096) -> dict:
