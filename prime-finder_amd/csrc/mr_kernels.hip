@@ -678,6 +678,7 @@ __device__ __forceinline__ void dec_value(Smem<LOGM> &sm, const Dev &D, int c, u
 
 // N = sum of coef * 10^exp over the candidate's terms; one workgroup each.
 // Ls_in (optional, per launch index) sets the slot's limb count.
+constexpr int BUILD_TERMS = 32;
 template <int LOGM>
 __global__ __launch_bounds__(THREADS) void build_kernel(Dev D, Twiddles T, Consts K,
                                                         const int64_t *terms, int tmax,
@@ -691,9 +692,34 @@ __global__ __launch_bounds__(THREADS) void build_kernel(Dev D, Twiddles T, Const
     for (int i = 0; i < C; i++) P[i] = Q[i] = 0u;
     const int64_t *tc = terms + (size_t)blockIdx.x * tmax * 2;
     if (Ls_in && threadIdx.x == 0) D.Ls[c] = Ls_in[blockIdx.x];
-    for (int t = 0; t < tmax; t++) {
-        const int64_t coef = tc[2 * t], ex = tc[2 * t + 1];
-        if (coef == 0) continue;
+    // Terms of one sign within 6 digits of each other share a power of ten (the
+    // digits of k, and of j, come as a term each; a power is up to 17 products):
+    // about 4 of 6.3 ms saved at 50 000 digits.
+    __shared__ int64_t gc[BUILD_TERMS], ge[BUILD_TERMS];
+    __shared__ int gn;
+    if (threadIdx.x == 0) {
+        const int64_t ten[7] = {1, 10, 100, 1000, 10000, 100000, 1000000};
+        int n = 0;
+        for (int t = 0; t < tmax; t++) {
+            const int64_t coef = tc[2 * t], ex = tc[2 * t + 1];
+            if (coef == 0) continue;
+            int g = 0;
+            for (; g < n; g++) {
+                const int64_t d = ex - ge[g];
+                if ((coef > 0) != (gc[g] > 0) || d > 6 || d < -6) continue;
+                const int64_t sum = d >= 0 ? gc[g] + coef * ten[d] : gc[g] * ten[-d] + coef;
+                if (sum >= 1 << LIMB_BITS || sum <= -(1 << LIMB_BITS)) continue;    // (mul_small_vec)
+                gc[g] = sum;
+                if (d < 0) ge[g] = ex;
+                break;
+            }
+            if (g == n) { gc[n] = coef; ge[n++] = ex; }
+        }
+        gn = n;
+    }
+    __syncthreads();
+    for (int t = 0; t < gn; t++) {
+        const int64_t coef = gc[t], ex = ge[t];
         pow5<LOGM>(sm, T, K, x, (long)ex, D.ysv + (size_t)c * G<LOGM>::YSV);
         const uint32_t mag = (uint32_t)(coef < 0 ? -coef : coef);
         if (mag != 1u) mul_small_vec<C>(x, mag, sm.sc);
@@ -1655,6 +1681,7 @@ bool ctx_try_alloc(mr_ctx *x, std::initializer_list<std::pair<void **, size_t>> 
 }
 
 constexpr int TMAX = 24;       // sparse decimal terms per candidate
+static_assert(TMAX <= BUILD_TERMS, "build_kernel groups them in LDS");
 
 // Limbs and log2 transform length for numbers of at most `bits` bits:
 // 24 L > bits, so that 2N < R = 2^(24 L).

@@ -107,3 +107,15 @@ def test_second_product_without_a_gap_below(gpu, tmp_path, digits):
     s.restore(tmp_path / "c")
     assert [bool(r.verdict) for r in sorted(s.run_all(), key=lambda r: r.tag)] == [bool(p[0]) for p in passed]
     s.close()
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_moduli_from_grouped_terms(gpu, which):
+    """N built from terms that share powers: digits of k and j apart, side by
+    side and interleaved, up to seven digits, at the top and at 10^0."""
+    cands = [(a, b, c, k, j, which) for a in (60, 300, 2000)
+             for b, c in ((a // 2, 20), (a // 2, a // 2 - 5), (a // 2, a // 2 - 1), (30, 31), (a - 9, 1), (12, 0))
+             for k, j in ((4096, 4095), (1000000, 999999), (1, 1000000), (101, 909), (999999, 7))]
+    ctx = gpu.MrContext(candidates=cands)
+    assert list(ctx.moduli()) == [gmp_build(*cd) for cd in cands]
+    ctx.close()
